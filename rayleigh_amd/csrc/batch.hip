@@ -19,7 +19,9 @@ struct raysht_batch {
     int precision = 0;
     std::vector<raysht_plan *> plans;
     raysht::prob_desc *d_desc = nullptr;
-    raysht::work_item *d_work[2][kSchedules] = {};  // [direction: 0 StP, 1 PtS][candidate]
+    // [direction: 0 StP, 1 PtS][candidate], of the batch's precision
+    raysht::work_item *d_work[2][kSchedules] = {};
+    raysht::fp64_item *d_work64[2][kSchedules] = {};
     int n_work[2][kSchedules] = {};
     int choice[2] = {0, 0};
 };
@@ -33,6 +35,9 @@ void batch_free(raysht_batch *b)
     if (b->d_desc) (void)hipFree(b->d_desc);
     for (auto &dir : b->d_work)
         for (work_item *w : dir)
+            if (w) (void)hipFree(w);
+    for (auto &dir : b->d_work64)
+        for (fp64_item *w : dir)
             if (w) (void)hipFree(w);
     delete b;
 }
@@ -48,10 +53,11 @@ bool distinct(const raysht_batch *b, int dir, int c)
 
 int launch_dir(raysht_batch *b, int dir, int c, const batch_io &io, hipStream_t st)
 {
-    work_item *w = b->d_work[dir][c];
     const int n = b->n_work[dir][c];
     if (b->precision == RAYSHT_FP64)
-        return dir == 0 ? launch_stp_fp64_batch(b->d_desc, io, w, n, st) : launch_pts_fp64_batch(b->d_desc, io, w, n, st);
+        return dir == 0 ? launch_stp_fp64_batch(io, b->d_work64[dir][c], n, st)
+                        : launch_pts_fp64_batch(io, b->d_work64[dir][c], n, st);
+    const work_item *w = b->d_work[dir][c];
     return dir == 0 ? launch_stp_split_batch(b->precision, b->d_desc, io, w, n, st)
                     : launch_pts_split_batch(b->precision, b->d_desc, io, w, n, st);
 }
@@ -107,10 +113,15 @@ int raysht_batch_create(raysht_batch **out, raysht_plan *const *plans, int n_pla
     int rc = upload(&b->d_desc, desc);
     for (int dir = 0; dir < 2 && rc == RAYSHT_OK; ++dir)
         for (int c = 0; c < kSchedules && rc == RAYSHT_OK; ++c) {
-            const std::vector<work_item> w =
-                fp64 ? fp64_work(cp, dir == 0, schedule(c)) : split_work(cp, dir == 0, schedule(c));
-            b->n_work[dir][c] = (int)w.size();
-            rc = upload(&b->d_work[dir][c], w);
+            if (fp64) {
+                const std::vector<fp64_item> w = fp64_work(cp, dir == 0, schedule(c));
+                b->n_work[dir][c] = (int)w.size();
+                rc = upload(&b->d_work64[dir][c], w);
+            } else {
+                const std::vector<work_item> w = split_work(cp, dir == 0, schedule(c));
+                b->n_work[dir][c] = (int)w.size();
+                rc = upload(&b->d_work[dir][c], w);
+            }
         }
     if (rc != RAYSHT_OK) {
         batch_free(b);

@@ -1269,7 +1269,7 @@ std::vector<work_item> split_work(const std::vector<const raysht_plan *> &plans,
         blocks.push_back(std::move(items));
         cost.push_back(b.item * nct);
     }
-    return deal_to_xcds(blocks, cost, o.xcd_groups);
+    return deal_to_xcds(blocks, cost, o.xcd_groups, work_item{-1, 0, 0, 0});
 }
 
 namespace {

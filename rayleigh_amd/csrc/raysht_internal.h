@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <vector>
@@ -27,17 +28,31 @@ struct dd_pair {
     double hi, lo;
 };
 
-// One unit of grouped-GEMM work: m-block mp, row tile start, column tile start, and in
-// `pad` the problem index (low 16 bits) and, for the FP64 PtS kernel, the tile shape (high
-// bits: 0 = the full tile, 1 / 2 / 3 = the half- / quarter- / three-quarter-height tile for
-// the last rows of an m-block).  The split kernels' items run every row tile of their
-// column tile.
+// One unit of grouped-GEMM work of the split kernels: m-block mp, column tile start, and in
+// `pad` the problem index.  An item runs every row tile of its column tile.
 struct work_item {
     int mp;
     int r0;
     int c0;
     int pad;
 };
+
+// One tile of the FP64 kernels: row tile start r0 (nodes for StP, parity-l for PtS), column
+// tile start c0 and everything the tile needs to start loading (one 64-byte scalar load
+// instead of a chain of four dependent ones through the problem's descriptor and offset
+// tables, each of which costs a memory latency while the tile's matrix cores are idle).
+// nl = 0 marks a padding item.
+struct fp64_item {
+    const double *te, *to;  // the m-block's even and odd table of the direction
+    long s_off, p_off;      // the m-block's offsets in the spectral and the hybrid array
+    int r0, c0;
+    int nl;                 // l_max - m + 1
+    int nt2, nrhs;          // N_theta / 2, columns
+    int prob;               // problem index: which input and output of the launch
+    int blocks;             // 16-row blocks of the tile, 1 .. 4
+    int pad;
+};
+static_assert(sizeof(fp64_item) == 64, "one cache line half per item");
 
 // Device state of the split-precision (BF16 slice) forms: the tables pre-split into
 // 1 KiB MFMA B-operand fragments (64 lanes x 8 BF16), the power-of-two scale exponent
@@ -91,7 +106,7 @@ struct raysht_plan {
     long *d_s_off = nullptr, *d_te_off = nullptr, *d_to_off = nullptr;
     int *d_mvals = nullptr;
     int *d_mp_of_m = nullptr;  // m -> mp, -1 where the plan has no such m
-    raysht::work_item *d_work_stp = nullptr, *d_work_pts = nullptr;
+    raysht::fp64_item *d_work_stp = nullptr, *d_work_pts = nullptr;
     int n_work_stp = 0, n_work_pts = 0;
     // staging buffers of the host-array entry points, allocated on first use
     double *d_stage_s = nullptr, *d_stage_p = nullptr;
@@ -159,10 +174,8 @@ int launch_plm_tables(raysht_plan *p, const double *d_x, const double *d_renorm,
 int launch_stp_fp64(raysht_plan *p, const double *s, double *p2, hipStream_t st);
 int launch_pts_fp64(raysht_plan *p, const double *p2, double *s, hipStream_t st);
 // grouped launches over the work items of several problems (descriptors in device memory)
-int launch_stp_fp64_batch(const prob_desc *d_desc, const batch_io &io, const work_item *work, int n_work,
-                          hipStream_t st);
-int launch_pts_fp64_batch(const prob_desc *d_desc, const batch_io &io, const work_item *work, int n_work,
-                          hipStream_t st);
+int launch_stp_fp64_batch(const batch_io &io, const fp64_item *work, int n_work, hipStream_t st);
+int launch_pts_fp64_batch(const batch_io &io, const fp64_item *work, int n_work, hipStream_t st);
 int launch_stp_split_batch(int precision, const prob_desc *d_desc, const batch_io &io, const work_item *work,
                            int n_work, hipStream_t st);
 int launch_pts_split_batch(int precision, const prob_desc *d_desc, const batch_io &io, const work_item *work,
@@ -176,12 +189,41 @@ struct sched_opts {
     bool half_tiles = true;
     bool xcd_groups = true;
 };
-std::vector<work_item> fp64_work(const std::vector<const raysht_plan *> &plans, bool stp, sched_opts o = {});
+std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, bool stp, sched_opts o = {});
 std::vector<work_item> split_work(const std::vector<const raysht_plan *> &plans, bool stp, sched_opts o = {});
-// deals per-block item lists to the XCDs (LPT over the block costs, blocks in the given
-// order) and interleaves them so that item i runs on XCD i % 8, or concatenates them
-std::vector<work_item> deal_to_xcds(const std::vector<std::vector<work_item>> &blocks,
-                                    const std::vector<double> &cost, bool xcd_groups);
+// Work items of one grouped launch.  Workgroups are dispatched to the 8 XCDs of the
+// chip round-robin by workgroup index, each XCD with its own L2.  Whole m-blocks are
+// assigned to XCDs (longest first, each to the least-loaded XCD) so that the tiles
+// of one m-block, which share its P_lm table and its input columns, run on one XCD
+// and hit in its L2; within an XCD the largest contractions come first.  The list
+// is interleaved so that workgroup b runs item b/8 of XCD b%8, padded with `empty`
+// items where XCD queues differ in length.  Without XCD groups the blocks' items are
+// concatenated in the same longest-first order.
+template <typename Item>
+std::vector<Item> deal_to_xcds(const std::vector<std::vector<Item>> &blocks, const std::vector<double> &cost,
+                               bool xcd_groups, const Item &empty)
+{
+    constexpr int kXcds = 8;
+    if (!xcd_groups) {
+        std::vector<Item> w;
+        for (const auto &b : blocks) w.insert(w.end(), b.begin(), b.end());
+        return w;
+    }
+    std::vector<std::vector<Item>> q(kXcds);
+    std::vector<double> load(kXcds, 0.0);
+    for (size_t i = 0; i < blocks.size(); ++i) {
+        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        q[x].insert(q[x].end(), blocks[i].begin(), blocks[i].end());
+        load[x] += cost[i];
+    }
+    size_t len = 0;
+    for (auto &v : q) len = std::max(len, v.size());
+    std::vector<Item> w(len * kXcds, empty);
+    for (size_t i = 0; i < len; ++i)
+        for (int x = 0; x < kXcds; ++x)
+            if (i < q[x].size()) w[i * kXcds + x] = q[x][i];
+    return w;
+}
 // allocates the device twiddle table of length-nphi FFTs (done by the first FFT call
 // otherwise; needed before a stream capture, which may not allocate)
 int fft_prepare(int nphi);

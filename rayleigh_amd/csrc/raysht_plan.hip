@@ -35,6 +35,16 @@ int device_upload(T **dst, const T *src, size_t n)
     return RAYSHT_OK;
 }
 
+// A P_lm table of n doubles and two zeros behind it: the 16-byte loads of the FP64 kernels
+// may start at the last value.
+int device_table(double **dst, size_t n)
+{
+    int rc = device_upload(dst, (const double *)nullptr, n + 2);
+    if (rc != RAYSHT_OK) return rc;
+    RAYSHT_HIP_TRY(hipMemset(*dst + n, 0, 2 * sizeof(double)));
+    return RAYSHT_OK;
+}
+
 template <typename T>
 void device_free(T *&ptr)
 {
@@ -47,43 +57,10 @@ int n_odd(int lmax, int m) { return (lmax - m + 1) / 2; }
 
 }  // namespace
 
-// Work items of one grouped launch.  Workgroups are dispatched to the 8 XCDs of the
-// chip round-robin by workgroup index, each XCD with its own L2.  Whole m-blocks are
-// assigned to XCDs (longest first, each to the least-loaded XCD) so that the tiles
-// of one m-block, which share its P_lm table and its input columns, run on one XCD
-// and hit in its L2; within an XCD the largest contractions come first.  The list
-// is interleaved so that workgroup b runs item b/8 of XCD b%8, padded with empty
-// items (mp = -1) where XCD queues differ in length.  Without XCD groups the blocks'
-// items are concatenated in the same longest-first order.
-std::vector<work_item> deal_to_xcds(const std::vector<std::vector<work_item>> &blocks,
-                                    const std::vector<double> &cost, bool xcd_groups)
-{
-    constexpr int kXcds = 8;
-    if (!xcd_groups) {
-        std::vector<work_item> w;
-        for (const auto &b : blocks) w.insert(w.end(), b.begin(), b.end());
-        return w;
-    }
-    std::vector<std::vector<work_item>> q(kXcds);
-    std::vector<double> load(kXcds, 0.0);
-    for (size_t i = 0; i < blocks.size(); ++i) {
-        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        q[x].insert(q[x].end(), blocks[i].begin(), blocks[i].end());
-        load[x] += cost[i];
-    }
-    size_t len = 0;
-    for (auto &v : q) len = std::max(len, v.size());
-    std::vector<work_item> w(len * kXcds, work_item{-1, 0, 0, 0});
-    for (size_t i = 0; i < len; ++i)
-        for (int x = 0; x < kXcds; ++x)
-            if (i < q[x].size()) w[i * kXcds + x] = q[x][i];
-    return w;
-}
-
 // The FP64 kernels' work list.  Inside an m-block the row tiles of one column tile are
 // consecutive, so they find the column tile's input in L2.  The m-blocks of several
-// problems share one list; `pad` holds the problem index and the tile shape.
-std::vector<work_item> fp64_work(const std::vector<const raysht_plan *> &plans, bool stp, sched_opts o)
+// problems share one list.
+std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, bool stp, sched_opts o)
 {
     const int tc = stp ? stp_tile_cols() : pts_tile_cols();
     const int tr = stp ? stp_tile_rows() : pts_tile_rows();
@@ -103,30 +80,39 @@ std::vector<work_item> fp64_work(const std::vector<const raysht_plan *> &plans, 
         if (a.prob != b.prob) return a.prob < b.prob;
         return plans[a.prob]->mvals[a.mp] < plans[b.prob]->mvals[b.mp];
     });
-    std::vector<std::vector<work_item>> blocks;
+    std::vector<std::vector<fp64_item>> blocks;
     std::vector<double> cost;
     for (const blk &b : order) {
         const raysht_plan *p = plans[b.prob];
         const int rows = stp ? p->nt2 : n_even(p->lmax, p->mvals[b.mp]);
         const int nrt = (rows + tr - 1) / tr, nct = (p->nrhs + tc - 1) / tc;
-        // PtS: a last row tile of at most a quarter, a half or three quarters of the height
-        // runs as that shape (shape code 2, 1 or 3)
-        const int rem = rows - (nrt - 1) * tr;
-        const int shape = (stp || !o.half_tiles) ? 0
-                          : rem <= tr / 4        ? 2
-                          : rem <= tr / 2        ? 1
-                          : rem <= 3 * tr / 4    ? 3
-                                                 : 0;
-        std::vector<work_item> items;
+        // 16-row blocks of the last row tile: as many as hold a row (StP always: its tiles end
+        // at the equator; PtS with half_tiles off runs full tiles)
+        const int rem = rows - (nrt - 1) * tr, full = tr / 16;
+        const int last = stp || o.half_tiles ? (rem + 15) / 16 : full;
+        fp64_item it{};
+        it.te = (stp ? p->d_pt_even : p->d_ip_even) + p->te_off[b.mp];
+        it.to = (stp ? p->d_pt_odd : p->d_ip_odd) + p->to_off[b.mp];
+        it.s_off = p->s_off[b.mp];
+        it.p_off = (long)b.mp * p->nrhs * p->nt;
+        it.nl = p->lmax - p->mvals[b.mp] + 1;
+        it.nt2 = p->nt2;
+        it.nrhs = p->nrhs;
+        it.prob = b.prob;
+        std::vector<fp64_item> items;
         // column tile outer, row tile inner: consecutive items share the column tile's
         // input (spectral columns for StP, hybrid columns for PtS) while it is in L2
         for (int c = 0; c < nct; ++c)
-            for (int r = 0; r < nrt; ++r)
-                items.push_back(work_item{b.mp, r * tr, c * tc, b.prob | ((r == nrt - 1 ? shape : 0) << 16)});
+            for (int r = 0; r < nrt; ++r) {
+                it.r0 = r * tr;
+                it.c0 = c * tc;
+                it.blocks = r == nrt - 1 ? last : full;
+                items.push_back(it);
+            }
         blocks.push_back(std::move(items));
-        cost.push_back(b.item * (nrt - (shape == 2 ? 0.75 : shape == 1 ? 0.5 : shape == 3 ? 0.25 : 0.0)) * nct);
+        cost.push_back(b.item * (nrt - 1 + (double)last / full) * nct);
     }
-    return deal_to_xcds(blocks, cost, o.xcd_groups);
+    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{});
 }
 
 void set_last_hip_error(hipError_t e, const char *what)
@@ -276,10 +262,6 @@ int plan_create(raysht_plan **out, int lmax, int ntheta, const int *m_values, in
         amp_dd[2 * m + 1] = amp_lo[m];
     }
 
-    std::vector<work_item> ws = fp64_work({p}, true), wp = fp64_work({p}, false);
-    p->n_work_stp = (int)ws.size();
-    p->n_work_pts = (int)wp.size();
-
     double *d_x = nullptr, *d_rn = nullptr, *d_amp = nullptr;
     const size_t ne_tot = p->te_off[n_m], no_tot = p->to_off[n_m];
     if ((rc = device_upload(&p->d_s_off, p->s_off.data(), p->s_off.size())) ||
@@ -287,12 +269,8 @@ int plan_create(raysht_plan **out, int lmax, int ntheta, const int *m_values, in
         (rc = device_upload(&p->d_to_off, p->to_off.data(), p->to_off.size())) ||
         (rc = device_upload(&p->d_mvals, p->mvals.data(), p->mvals.size())) ||
         (rc = device_upload(&p->d_mp_of_m, seen.data(), seen.size())) ||
-        (rc = device_upload(&p->d_work_stp, ws.data(), ws.size())) ||
-        (rc = device_upload(&p->d_work_pts, wp.data(), wp.size())) ||
-        (rc = device_upload(&p->d_pt_even, (const double *)nullptr, ne_tot)) ||
-        (rc = device_upload(&p->d_ip_even, (const double *)nullptr, ne_tot)) ||
-        (rc = device_upload(&p->d_pt_odd, (const double *)nullptr, std::max<size_t>(no_tot, 1))) ||
-        (rc = device_upload(&p->d_ip_odd, (const double *)nullptr, std::max<size_t>(no_tot, 1))) ||
+        (rc = device_table(&p->d_pt_even, ne_tot)) || (rc = device_table(&p->d_ip_even, ne_tot)) ||
+        (rc = device_table(&p->d_pt_odd, no_tot)) || (rc = device_table(&p->d_ip_odd, no_tot)) ||
         (rc = device_upload(&d_x, x_dd.data(), x_dd.size())) ||
         (rc = device_upload(&d_rn, rn_dd.data(), rn_dd.size())) ||
         (rc = device_upload(&d_amp, amp_dd.data(), amp_dd.size()))) {
@@ -302,7 +280,15 @@ int plan_create(raysht_plan **out, int lmax, int ntheta, const int *m_values, in
         raysht_plan_destroy(p);
         return rc;
     }
-    rc = launch_plm_tables(p, d_x, d_rn, d_amp, nullptr);
+    // the FP64 kernels' work lists hold the tables' addresses
+    if (precision == RAYSHT_FP64) {
+        const std::vector<fp64_item> ws = fp64_work({p}, true), wp = fp64_work({p}, false);
+        p->n_work_stp = (int)ws.size();
+        p->n_work_pts = (int)wp.size();
+        if ((rc = device_upload(&p->d_work_stp, ws.data(), ws.size())) == RAYSHT_OK)
+            rc = device_upload(&p->d_work_pts, wp.data(), wp.size());
+    }
+    if (rc == RAYSHT_OK) rc = launch_plm_tables(p, d_x, d_rn, d_amp, nullptr);
     if (rc == RAYSHT_OK && hipDeviceSynchronize() != hipSuccess) rc = RAYSHT_EHIP;
     device_free(d_x);
     device_free(d_rn);
