@@ -85,11 +85,12 @@ std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, 
     for (const blk &b : order) {
         const raysht_plan *p = plans[b.prob];
         const int rows = stp ? p->nt2 : n_even(p->lmax, p->mvals[b.mp]);
-        const int nrt = (rows + tr - 1) / tr, nct = (p->nrhs + tc - 1) / tc;
-        // 16-row blocks of the last row tile: as many as hold a row (StP always: its tiles end
-        // at the equator; PtS with half_tiles off runs full tiles)
-        const int rem = rows - (nrt - 1) * tr, full = tr / 16;
-        const int last = stp || o.half_tiles ? (rem + 15) / 16 : full;
+        const int nct = (p->nrhs + tc - 1) / tc;
+        // The rows in 16-row blocks, dealt evenly to the fewest tiles (13 blocks: 4 + 3 + 3 + 3
+        // and not 4 + 4 + 4 + 1): a tile of one block reads as much input as one of four.
+        const int full = tr / 16, nblk = (rows + 15) / 16, nrt = (nblk + full - 1) / full;
+        // (StP always: its tiles end at the equator.  PtS with half_tiles off runs full tiles.)
+        const bool exact = stp || o.half_tiles;
         fp64_item it{};
         it.te = (stp ? p->d_pt_even : p->d_ip_even) + p->te_off[b.mp];
         it.to = (stp ? p->d_pt_odd : p->d_ip_odd) + p->to_off[b.mp];
@@ -103,16 +104,30 @@ std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, 
         // column tile outer, row tile inner: consecutive items share the column tile's
         // input (spectral columns for StP, hybrid columns for PtS) while it is in L2
         for (int c = 0; c < nct; ++c)
-            for (int r = 0; r < nrt; ++r) {
-                it.r0 = r * tr;
+            for (int r = 0, at = 0; r < nrt; ++r) {
                 it.c0 = c * tc;
-                it.blocks = r == nrt - 1 ? last : full;
+                it.r0 = 16 * at;
+                it.blocks = exact ? nblk / nrt + (r < nblk % nrt ? 1 : 0) : full;
+                at += it.blocks;
                 items.push_back(it);
             }
         blocks.push_back(std::move(items));
-        cost.push_back(b.item * (nrt - 1 + (double)last / full) * nct);
+        cost.push_back(b.item * (exact ? (double)nblk / full : nrt) * nct);
     }
-    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{});
+    // In a long launch heavy and light m-blocks alternate, so that tiles bound by the matrix
+    // cores (long contractions) share the CUs with tiles bound by memory (short ones, which
+    // otherwise all run together at the end).  In a short one the longest tiles go first:
+    // the tail they leave would cost more.  Measured (StP / PtS ms): l_max = 511, N_r = 192, 8
+    // fields, 72 / 51 rounds: 6.00 / 6.25 -> 5.91 / 6.15; l_max = 255, N_r = 128, 12 / 9 rounds:
+    // 0.648 / 0.646 -> 0.644 / 0.639; a batch of 12 problems, 7 / 5 rounds: 0.546 / 0.547 ->
+    // 0.552 / 0.564.
+    double total = 0.0, longest = 0.0;
+    for (size_t i = 0; i < order.size(); ++i) {
+        total += cost[i];
+        longest = std::max(longest, order[i].item);
+    }
+    constexpr double kSlots = 512.0, kMixRounds = 8.0;  // two workgroups on each of 256 CUs
+    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{}, total >= kMixRounds * kSlots * longest);
 }
 
 void set_last_hip_error(hipError_t e, const char *what)
