@@ -6,17 +6,15 @@
 // many matrices go in one launch, one workgroup per matrix (factorisation) or per
 // matrix and chunk of its right-hand sides (solve).
 //
-// Factorisation: the unblocked right-looking algorithm of dgetf2 -- pivot = first row of
-// largest |a_ik| (a workgroup reduction), row swap, subdiagonal scaled by the pivot's
-// reciprocal, rank-1 update of the trailing block -- with products and sums rounded
-// separately.  The matrix stays in global memory (L2); per column the pivot row goes to
-// LDS and each thread sweeps whole rows of the trailing block (coalesced across threads,
-// sixteen loads in flight per thread).
+// Factorisation: the right-looking algorithm of dgetf2 -- pivot = first row of largest
+// |a_ik|, row swap, subdiagonal scaled by the pivot's reciprocal, rank-1 update of the
+// trailing block -- with products and sums rounded separately, in panels.
 // Solve: the row interchanges, the unit lower and the upper triangular solves in the
 // column order of the reference BLAS dtrsm (column j final, then subtracted from the rows
 // below / above it).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "raysht_internal.h"
 
@@ -25,7 +23,6 @@ namespace {
 
 constexpr int kLuThreads = 256;
 constexpr int kLuMaxN = 1024;
-constexpr int kLuBatch = 16;  // row loads in flight per thread in the factorisation sweep (4: 1.3x slower)
 
 // Workgroup order of the solves.  Workgroups go to the 8 XCDs round-robin by linear id, so
 // XCD k runs ids k, k + 8, k + 16, ...; its r-th workgroup takes column block r % ncb of
@@ -55,280 +52,302 @@ inline bool solve_grid_fits(int ncb, int nbatch, int grouped, int threads)
     return solve_grid(ncb, nbatch, grouped) * threads < (1L << 32);
 }
 
-__global__ __launch_bounds__(kLuThreads) void lu_decompose_kernel(int n, double *__restrict__ mats,
-                                                                  int *__restrict__ pivots, int *__restrict__ infos)
+// Factorisation, one workgroup per matrix, panels of kLuNB columns.  A thread owns one row of
+// the panel and holds its kLuNB values in registers for all of the panel's column steps.  An
+// interchange moves nothing: a thread keeps the position its row stands at, and only these
+// change.  Per step each wave finds its candidate (largest |a|, lowest position among equals;
+// DPP lane moves) and leaves the whole candidate row in LDS, so after one barrier every
+// thread knows the pivot and has its row, scales its own value and updates its own row.  Then
+// the rows go back to memory at their positions, the rest of the matrix takes the panel's
+// interchanges (a wave per column, at most 32 rows move), U12 is formed by a thread per
+// column and the trailing block by register tiles that apply the panel's updates
+// k = k0 .. k0 + kLuNB - 1 one after the other.  Products and sums are rounded separately and a
+// zero u_kj skipped (dger), so every element sees the operations of dgetf2 in its order and
+// the factors are its doubles.
+// What it waits for is the column steps (a chain of a reduction, a barrier, LDS reads and a
+// reciprocal, about a third of n = 256), then the passes over the trailing block, which the
+// caches and FP64 vector arithmetic share (matrix instructions would fuse the product into the
+// sum).  256 matrices of n = 64, 128, 256: 0.13, 0.33, 0.87 ms; 128 of n = 512: 3.3 ms, 32 of
+// n = 1000: 19 ms; steps
+// that go through global memory (the search, the interchange of the whole row, the update of
+// the panel) took 0.31, 0.67, 2.39, 9.1 and
+// 45 ms.  Panels of 32 need a step code of 137 KB, more than the
+// instruction cache, and were slower at every n.
+constexpr int kLuNB = 16;
+constexpr int kLuChunk = 256;  // rows of L21 and columns of U12 in LDS at a time
+
+// the largest m of the wave (no NaN), in every lane
+__device__ __forceinline__ double lu_wave_max(double m)
 {
-#pragma clang fp contract(off)
-    __shared__ double s_val[kLuThreads];
-    __shared__ int s_idx[kLuThreads];
-    __shared__ double rowk[kLuMaxN];  // the pivot row, columns k + 1 .. n - 1
-    double *a = mats + (long)blockIdx.x * n * n;
-    int *piv = pivots + (long)blockIdx.x * n;
-    const int tid = threadIdx.x;
-    const double sfmin = 2.2250738585072014e-308;
-    int info = 0;
-    for (int k = 0; k < n; ++k) {
-        // pivot: the first row of largest |a_ik|, i >= k
-        double best = -1.0;
-        int bi = n;
-        for (int i = k + tid; i < n; i += kLuThreads) {
-            const double v = fabs(a[i + (long)k * n]);
-            if (v > best) {
-                best = v;
-                bi = i;
-            }
-        }
-        s_val[tid] = best;
-        s_idx[tid] = bi;
-        __syncthreads();
-        for (int s = kLuThreads / 2; s > 0; s >>= 1) {
-            if (tid < s) {
-                const double v = s_val[tid + s];
-                const int j = s_idx[tid + s];
-                if (v > s_val[tid] || (v == s_val[tid] && j < s_idx[tid])) {
-                    s_val[tid] = v;
-                    s_idx[tid] = j;
-                }
-            }
-            __syncthreads();
-        }
-        // idamax: a NaN a_kk is kept (nothing compares larger than it), as is row k of a
-        // column of NaNs; NaNs below the diagonal are passed over
-        const int p = (s_idx[0] >= n || isnan(a[k + (long)k * n])) ? k : s_idx[0];
-        const double pv = a[p + (long)k * n];
-        __syncthreads();  // every thread has read the pivot before the swap moves it
-        if (tid == 0) piv[k] = p + 1;
-        if (pv != 0.0) {
-            if (p != k)
-                for (int j = tid; j < n; j += kLuThreads) {
-                    const double t = a[k + (long)j * n];
-                    a[k + (long)j * n] = a[p + (long)j * n];
-                    a[p + (long)j * n] = t;
-                }
-        } else if (info == 0) {
-            info = k + 1;
-        }
-        __syncthreads();
-        for (int j = k + 1 + tid; j < n; j += kLuThreads) rowk[j] = a[k + (long)j * n];
-        __syncthreads();
-        // each thread: its rows i > k -- scale a_ik by the pivot's reciprocal, then sweep the
-        // row, a_ij + a_ik (-a_kj), four columns at a time (loads issued together)
-        const double r = pv != 0.0 && fabs(pv) >= sfmin ? 1.0 / pv : 0.0;
-        for (int i = k + 1 + tid; i < n; i += kLuThreads) {
-            double lik = a[i + (long)k * n];
-            if (pv != 0.0) {
-                lik = fabs(pv) >= sfmin ? lik * r : lik / pv;
-                a[i + (long)k * n] = lik;
-            }
-            double *ai = a + i;
-            int j = k + 1;
-            for (; j + kLuBatch - 1 < n; j += kLuBatch) {
-                double v[kLuBatch];
-#pragma unroll
-                for (int u = 0; u < kLuBatch; ++u) v[u] = ai[(long)(j + u) * n];
-#pragma unroll
-                for (int u = 0; u < kLuBatch; ++u) {
-                    const double y = rowk[j + u];
-                    if (y != 0.0) ai[(long)(j + u) * n] = v[u] + lik * -y;
-                }
-            }
-            for (; j < n; ++j) {
-                const double y = rowk[j];
-                if (y != 0.0) ai[(long)j * n] = ai[(long)j * n] + lik * -y;
-            }
-        }
-        __syncthreads();
-    }
-    if (tid == 0) infos[blockIdx.x] = info;
+    auto step = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        const long b = __builtin_bit_cast(long, m);
+        const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, C, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), C, 0xf, 0xf, false);
+        m = fmax(m, __builtin_bit_cast(double, ((long)hi << 32) | (unsigned)lo));
+    };
+    step(std::integral_constant<int, 0x111>{});  // row_shr 1, 2, 4, 8: lane 15 of a row has its row's
+    step(std::integral_constant<int, 0x112>{});
+    step(std::integral_constant<int, 0x114>{});
+    step(std::integral_constant<int, 0x118>{});
+    step(std::integral_constant<int, 0x142>{});  // row_bcast 15, 31: lane 63 has the wave's
+    step(std::integral_constant<int, 0x143>{});
+    const long b = __builtin_bit_cast(long, m);
+    const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __builtin_bit_cast(double, ((long)hi << 32) | (unsigned)lo);
 }
 
-// Blocked form of the same factorisation (n > kLuNB): panels of kLuNB columns.  Within a
-// panel, each column step is the one above (pivot, interchange of the whole row, scaling),
-// with the rank-1 update restricted to the panel's columns; the rest of the matrix then
-// takes the panel's kLuNB updates at once: U12 (the panel's rows, later columns) by forward
-// substitution with L11, and the trailing block by register tiles that apply the updates
-// k = k0 .. k0 + kLuNB - 1 one after the other, a_ij + l_ik (-u_kj), product and sum rounded
-// separately and skipped where u_kj = 0 (dger).  Every element thus sees the same
-// operations, in the same order, as in the column-by-column sweep (an interchange moves a
-// row's multipliers with it, so applying the panel's updates after the panel's
-// interchanges is the same arithmetic), and the factors are bit-identical; but the
-// trailing block is read and written once per panel instead of once per column, which
-// was 0.72 GB per matrix of n = 512.
-constexpr int kLuNB = 32;  // panel width
-constexpr int kLuT = 64;   // trailing-update chunk: kLuT x kLuT, 4 x 4 per thread
-
-__device__ __forceinline__ void lu_pivot_reduce(double &best, int &bi, double *s_val, int *s_idx)
+// f(0), f(1), ... with compile-time arguments: register arrays are indexed by constants however
+// long the unrolled code is
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_steps(F &&f)
 {
-    // first row of the largest |a|: (value, index) pairs ordered by value, then by lower index
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const double v = __shfl_down(best, off, 64);
-        const int j = __shfl_down(bi, off, 64);
-        if (v > best || (v == best && j < bi)) {
-            best = v;
-            bi = j;
-        }
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-        s_val[wave] = best;
-        s_idx[wave] = bi;
-    }
-    __syncthreads();
-    best = s_val[0];
-    bi = s_idx[0];
-#pragma unroll
-    for (int w = 1; w < kLuThreads / 64; ++w) {
-        const double v = s_val[w];
-        const int j = s_idx[w];
-        if (v > best || (v == best && j < bi)) {
-            best = v;
-            bi = j;
-        }
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_steps<I + 1, N>(f);
     }
 }
 
-__global__ __launch_bounds__(kLuThreads) void lu_decompose_blocked_kernel(int n, double *__restrict__ mats,
-                                                                          int *__restrict__ pivots,
-                                                                          int *__restrict__ infos)
+// LDS of one workgroup: two sets of candidate rows, L11, the moves, U12 and L21 chunks
+__host__ __device__ inline int lu_chunk(int n) { return n < kLuChunk ? n : kLuChunk; }
+__host__ __device__ inline int lu_ld(int n) { return lu_chunk(n) | 1; }
+template <int NT>
+size_t lu_lds_bytes(int n)
+{
+    constexpr int W = NT / 64;
+    return sizeof(double) * (2 * W * (kLuNB + 1) + kLuNB * (kLuNB + 2) + 2 * kLuNB * (size_t)lu_ld(n)) +
+           sizeof(int) * (2 * W + 2 * 64 + 2);
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void lu_decompose_kernel(int n, double *__restrict__ mats, int *__restrict__ pivots,
+                                                          int *__restrict__ infos)
 {
 #pragma clang fp contract(off)
-    __shared__ double s_val[kLuThreads / 64];
-    __shared__ int s_idx[kLuThreads / 64];
-    __shared__ double rowk[kLuNB];            // the pivot row within the panel
-    __shared__ double s_l[kLuNB][kLuT];       // L21 chunk [k][row]
-    __shared__ double s_u[kLuNB][kLuT];       // U12 chunk [k][column]
-    __shared__ double s_l11[kLuNB][kLuNB + 1];  // L11 [i][k]
+    constexpr int W = NT / 64, J = NT > 512 ? 4 : 8;
+    extern __shared__ double lu_lds[];
+    const int ld = lu_ld(n), chunk = lu_chunk(n);
+    double *s_row = lu_lds;                              // [2][W][kLuNB] candidate rows
+    double *s_val = s_row + 2 * W * kLuNB;               // [2][W] their |a|
+    double *s_l11 = s_val + 2 * W;                       // [k][row], rows kLuNB + 2 apart
+    double *s_u = s_l11 + kLuNB * (kLuNB + 2);           // [k][column]
+    double *s_l = s_u + kLuNB * ld;                      // [k][row]
+    int *s_pos = reinterpret_cast<int *>(s_l + kLuNB * ld);  // [2][W] the candidates' positions
+    int *s_src = s_pos + 2 * W, *s_dst = s_src + 64, *s_cnt = s_dst + 64, *s_zero = s_cnt + 1;
     double *a = mats + (long)blockIdx.x * n * n;
     int *piv = pivots + (long)blockIdx.x * n;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const double sfmin = 2.2250738585072014e-308;
+    constexpr int kNone = 1 << 30;
     int info = 0;
     for (int k0 = 0; k0 < n; k0 += kLuNB) {
-        const int kend = min(n, k0 + kLuNB);
-        // ---- the panel, column by column
-        for (int k = k0; k < kend; ++k) {
-            double best = -1.0;
-            int bi = n;
-            for (int i = k + tid; i < n; i += kLuThreads) {
-                const double v = fabs(a[i + (long)k * n]);
-                if (v > best) {
-                    best = v;
-                    bi = i;
+        const int nb = min(kLuNB, n - k0), kend = k0 + nb, row = k0 + tid;
+        // ---- the panel
+        double v[kLuNB];
+#pragma unroll
+        for (int j = 0; j < kLuNB; ++j) v[j] = row < n && j < nb ? a[row + (long)(k0 + j) * n] : 0.0;
+        int pos = row < n ? row : -1;
+        if (tid == 0) *s_cnt = 0;
+        static_steps<0, kLuNB>([&](auto step) {
+            constexpr int kk = decltype(step)::value, par = kk & 1;
+            if (kk >= nb) return;
+            const int k = k0 + kk;
+            // idamax: NaNs below the diagonal are passed over, a NaN a_kk is kept (it beats
+            // everything, an infinity by its lower key)
+            const double x = v[kk];
+            const bool in = pos >= k, nan = isnan(x);
+            const double m = !in || (nan && pos != k) ? -1.0 : nan ? HUGE_VAL : fabs(x);
+            const int key = !in || (nan && pos != k) ? kNone : nan ? -1 : pos;
+            const double wm = lu_wave_max(m);
+            unsigned long long eq = __ballot(m == wm);
+            int bl = __builtin_ctzll(eq);
+            if (wm >= 0.0)  // below: no row of this wave is a candidate
+                for (eq &= eq - 1; eq != 0; eq &= eq - 1) {  // equal candidates: the lowest position
+                    const int l2 = __builtin_ctzll(eq);
+                    if (__builtin_amdgcn_readlane(key, l2) < __builtin_amdgcn_readlane(key, bl)) bl = l2;
+                }
+            if (lane == bl) {
+                double *r = s_row + (par * W + wave) * kLuNB;
+#pragma unroll
+                for (int j = kk; j < kLuNB; ++j) r[j] = v[j];
+                s_val[par * W + wave] = m;
+                s_pos[par * W + wave] = key;
+            }
+            __syncthreads();  // the other set of rows was read before the previous step's barrier
+            int bw = 0, bk = s_pos[par * W];
+            double bv = s_val[par * W];
+#pragma unroll
+            for (int w = 1; w < W; ++w) {
+                const double ov = s_val[par * W + w];
+                const int ok = s_pos[par * W + w];
+                if (ov > bv || (ov == bv && ok < bk)) {
+                    bv = ov;
+                    bk = ok;
+                    bw = w;
                 }
             }
-            lu_pivot_reduce(best, bi, s_val, s_idx);
-            // idamax: a NaN a_kk is kept, as is row k of a column of NaNs
-            const int p = (bi >= n || isnan(a[k + (long)k * n])) ? k : bi;
-            const double pv = a[p + (long)k * n];
-            __syncthreads();  // every thread has read the pivot before the swap moves it
+            const int p = bk < 0 || bk == kNone ? k : bk;
+            const double *r = s_row + (par * W + __builtin_amdgcn_readfirstlane(bw)) * kLuNB;
+            const double pv = r[kk];
             if (tid == 0) piv[k] = p + 1;
             if (pv != 0.0) {
-                if (p != k)
-                    for (int j = tid; j < n; j += kLuThreads) {
-                        const double t = a[k + (long)j * n];
-                        a[k + (long)j * n] = a[p + (long)j * n];
-                        a[p + (long)j * n] = t;
-                    }
+                pos = pos == p ? k : pos == k ? p : pos;
             } else if (info == 0) {
                 info = k + 1;
             }
-            __syncthreads();
-            if (tid < kend - k - 1) rowk[tid] = a[k + (long)(k + 1 + tid) * n];
-            __syncthreads();
-            const double r = pv != 0.0 && fabs(pv) >= sfmin ? 1.0 / pv : 0.0;
-            for (int i = k + 1 + tid; i < n; i += kLuThreads) {
-                double lik = a[i + (long)k * n];
-                if (pv != 0.0) {
-                    lik = fabs(pv) >= sfmin ? lik * r : lik / pv;
-                    a[i + (long)k * n] = lik;
-                }
-                double *ai = a + i;
-                for (int j = k + 1; j < kend; ++j) {
-                    const double y = rowk[j - k - 1];
-                    if (y != 0.0) ai[(long)j * n] = ai[(long)j * n] + lik * -y;
+            if (pos > k) {
+                double lik = x;
+                if (pv != 0.0) lik = fabs(pv) >= sfmin ? x * (1.0 / pv) : x / pv;
+                v[kk] = lik;
+#pragma unroll
+                for (int j = kk + 1; j < kLuNB; ++j) {
+                    const double y = r[j], upd = v[j] + lik * -y;
+                    v[j] = y != 0.0 ? upd : v[j];
                 }
             }
-            __syncthreads();
-        }
-        if (kend >= n) break;
-        // ---- U12: rows k0 .. k0 + kLuNB - 1 of the later columns, forward substitution
-        for (int e = tid; e < kLuNB * kLuNB; e += kLuThreads) {
-            const int i = e % kLuNB, kk = e / kLuNB;
-            s_l11[i][kk] = a[k0 + i + (long)(k0 + kk) * n];
-        }
-        __syncthreads();
-        // a half wave per four columns: lane i % 32 holds row k0 + i of each, and step kk takes
-        // u_kk from lane kk of its half (the row-kk value is final once steps 0 .. kk - 1 are
-        // done); the four columns' shuffle chains are independent, so their latencies overlap
-        for (int j0 = kend + 4 * (tid / 32); j0 < n; j0 += 4 * (kLuThreads / 32)) {
-            const int i = tid % 32, half = tid & 32;
-            double u[4];
+        });
+        // ---- back to memory at the rows' positions; L11 and the moves to LDS
+        if (row < n) {
 #pragma unroll
-            for (int cc = 0; cc < 4; ++cc) u[cc] = j0 + cc < n ? a[k0 + i + (long)(j0 + cc) * n] : 0.0;
-            for (int kk = 0; kk < kLuNB - 1; ++kk) {
-                const double lik = s_l11[i][kk];
+            for (int j = 0; j < kLuNB; ++j)
+                if (j < nb) a[pos + (long)(k0 + j) * n] = v[j];
+            if (pos < kend) {
 #pragma unroll
-                for (int cc = 0; cc < 4; ++cc) {
-                    const double y = __shfl(u[cc], half | kk, 64);
-                    const double upd = u[cc] + lik * -y;
-                    u[cc] = (i > kk && y != 0.0) ? upd : u[cc];
-                }
+                for (int j = 0; j < kLuNB; ++j) s_l11[j * (kLuNB + 2) + pos - k0] = v[j];
             }
-#pragma unroll
-            for (int cc = 0; cc < 4; ++cc)
-                if (j0 + cc < n) a[k0 + i + (long)(j0 + cc) * n] = u[cc];
+            if (pos != row) {
+                const int at = atomicAdd(s_cnt, 1);  // a step moves at most two rows: at most 32
+                s_src[at] = row;
+                s_dst[at] = pos;
+            }
         }
         __syncthreads();
-        // ---- the trailing block, kLuT x kLuT chunks
-        const int tr = tid / 16, tc = tid % 16;
-        for (int r0 = kend; r0 < n; r0 += kLuT) {
-            for (int e = tid; e < kLuNB * kLuT; e += kLuThreads) {
-                const int row = e % kLuT, kk = e / kLuT;
-                s_l[kk][row] = r0 + row < n ? a[r0 + row + (long)(k0 + kk) * n] : 0.0;
+        // ---- the interchanges in the other columns, a wave per column, eight in flight
+        const int cnt = *s_cnt, others = n - nb;
+        if (cnt > 0) {
+            const int src = lane < cnt ? s_src[lane] : 0, dst = lane < cnt ? s_dst[lane] : 0;
+            constexpr int U = 8;
+            for (int q0 = wave; q0 < others; q0 += U * W) {
+                double t[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int q = q0 + u * W, col = q < k0 ? q : q + nb;
+                    t[u] = q < others && lane < cnt ? a[src + (long)col * n] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int q = q0 + u * W, col = q < k0 ? q : q + nb;
+                    if (q < others && lane < cnt) a[dst + (long)col * n] = t[u];
+                }
             }
-            for (int c0 = kend; c0 < n; c0 += kLuT) {
-                for (int e = tid; e < kLuNB * kLuT; e += kLuThreads) {
-                    const int col = e / kLuNB, kk = e % kLuNB;
-                    s_u[kk][col] = c0 + col < n ? a[k0 + kk + (long)(c0 + col) * n] : 0.0;
+        }
+        if (kend >= n) break;  // nb = kLuNB from here on
+        for (int c0 = kend; c0 < n; c0 += chunk) {
+            const int nc = min(chunk, n - c0);
+            __syncthreads();
+            // ---- U12 of this chunk: rows k0 .. k0 + kLuNB - 1, a thread per column
+            for (int e = tid; e < kLuNB * nc; e += NT) {
+                const int i = e % kLuNB, c = e / kLuNB;
+                s_u[i * ld + c] = a[k0 + i + (long)(c0 + c) * n];
+            }
+            if (tid == 0) *s_zero = 0;
+            __syncthreads();
+            for (int c = tid; c < nc; c += NT) {
+                double u[kLuNB];
+                bool zero = false;
+#pragma unroll
+                for (int i = 0; i < kLuNB; ++i) u[i] = s_u[i * ld + c];
+                static_steps<0, kLuNB>([&](auto step) {
+                    constexpr int kk = decltype(step)::value;
+                    const double y = u[kk];
+                    zero |= y == 0.0;
+#pragma unroll
+                    for (int i = kk + 1; i < kLuNB; ++i) {
+                        const double upd = u[i] + s_l11[kk * (kLuNB + 2) + i] * -y;
+                        u[i] = y != 0.0 ? upd : u[i];
+                    }
+                });
+#pragma unroll
+                for (int i = 0; i < kLuNB; ++i) s_u[i * ld + c] = u[i];
+                if (zero) *s_zero = 1;
+            }
+            __syncthreads();
+            for (int e = tid; e < kLuNB * nc; e += NT) {
+                const int i = e % kLuNB, c = e / kLuNB;
+                a[k0 + i + (long)(c0 + c) * n] = s_u[i * ld + c];
+            }
+            // ---- the trailing block: a wave per tile of 64 rows x 4 J columns, lane (li, lg) on rows
+            // li + 16 i and columns lg + 4 j (J = 8; 4 where 16 waves leave a thread 128 registers)
+            const bool any_zero = *s_zero != 0;
+            for (int r0 = kend; r0 < n; r0 += chunk) {
+                const int nr = min(chunk, n - r0);
+                if (r0 > kend) __syncthreads();
+                if (pos >= r0 && pos < r0 + nr) {
+#pragma unroll
+                    for (int j = 0; j < kLuNB; ++j) s_l[j * ld + pos - r0] = v[j];
                 }
                 __syncthreads();
-                const int i0 = r0 + 4 * tr, j0 = c0 + 4 * tc;
-                double t[4][4];
+                const int nrt = (nr + 63) / 64, nct = (nc + 4 * J - 1) / (4 * J);
+                const int li = lane & 15, lg = lane >> 4;
+                for (int tile = wave; tile < nrt * nct; tile += W) {
+                    const int tr = 64 * (tile % nrt), tc = 4 * J * (tile / nrt);
+                    double t[4][J];
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
+                    for (int j = 0; j < J; ++j)
 #pragma unroll
-                    for (int rr = 0; rr < 4; ++rr)
-                        t[rr][c] = (i0 + rr < n && j0 + c < n) ? a[i0 + rr + (long)(j0 + c) * n] : 0.0;
-#pragma unroll 4
-                for (int kk = 0; kk < kLuNB; ++kk) {
-                    double l[4], y[4];
-#pragma unroll
-                    for (int rr = 0; rr < 4; ++rr) l[rr] = s_l[kk][4 * tr + rr];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) y[c] = s_u[kk][4 * tc + c];
-                    // dger skips a zero u_kj: a select, not a branch per column
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const bool nz = y[c] != 0.0;
-#pragma unroll
-                        for (int rr = 0; rr < 4; ++rr) {
-                            const double upd = t[rr][c] + l[rr] * -y[c];
-                            t[rr][c] = nz ? upd : t[rr][c];
+                        for (int i = 0; i < 4; ++i) {
+                            const int rr = tr + li + 16 * i, cc = tc + lg + 4 * j;
+                            t[i][j] = rr < nr && cc < nc ? a[r0 + rr + (long)(c0 + cc) * n] : 0.0;
                         }
-                    }
+                    // rows and columns past the chunk take its last one's; their results are not
+                    // stored
+                    int ol[4], ou[J];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) ol[i] = min(tr + li + 16 * i, nr - 1);
+#pragma unroll
+                    for (int j = 0; j < J; ++j) ou[j] = min(tc + lg + 4 * j, nc - 1);
+                    auto sweep = [&](auto skip) {
+#pragma unroll 2
+                        for (int kk = 0; kk < kLuNB; ++kk) {
+                            double l[4], y[J];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) l[i] = s_l[kk * ld + ol[i]];
+#pragma unroll
+                            for (int j = 0; j < J; ++j) y[j] = s_u[kk * ld + ou[j]];
+#pragma unroll
+                            for (int j = 0; j < J; ++j)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    const double upd = t[i][j] + l[i] * -y[j];
+                                    if constexpr (decltype(skip)::value) t[i][j] = y[j] != 0.0 ? upd : t[i][j];
+                                    else t[i][j] = upd;
+                                }
+                        }
+                    };
+                    if (any_zero) sweep(std::true_type{});
+                    else sweep(std::false_type{});
+#pragma unroll
+                    for (int j = 0; j < J; ++j)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int rr = tr + li + 16 * i, cc = tc + lg + 4 * j;
+                            if (rr < nr && cc < nc) a[r0 + rr + (long)(c0 + cc) * n] = t[i][j];
+                        }
                 }
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-#pragma unroll
-                    for (int rr = 0; rr < 4; ++rr)
-                        if (i0 + rr < n && j0 + c < n) a[i0 + rr + (long)(j0 + c) * n] = t[rr][c];
-                __syncthreads();  // the chunk's U12 and (at the row chunk's end) L21 are free again
             }
         }
         __syncthreads();
     }
     if (tid == 0) infos[blockIdx.x] = info;
+}
+
+template <int NT>
+int launch_lu_decompose(int n, int nbatch, double *mats, int *pivots, int *info, hipStream_t st)
+{
+    hipLaunchKernelGGL(lu_decompose_kernel<NT>, dim3((unsigned)nbatch), dim3(NT), lu_lds_bytes<NT>(n), st, n, mats,
+                       pivots, info);
+    RAYSHT_HIP_TRY(hipGetLastError());
+    return RAYSHT_OK;
 }
 
 // Solve with the right-hand sides in registers: G lanes of a wave own CPL columns, lane
@@ -901,14 +920,13 @@ int raysht_lu_decompose_full(int n, int nbatch, double *mats, int *pivots, int *
     if (n < 1 || nbatch < 0 || (nbatch > 0 && (!mats || !pivots || !info))) return RAYSHT_EINVAL;
     if (n > kLuMaxN) return RAYSHT_EUNSUPPORTED;
     if (nbatch == 0) return RAYSHT_OK;
-    if (n > kLuNB)
-        hipLaunchKernelGGL(lu_decompose_blocked_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), 0,
-                           reinterpret_cast<hipStream_t>(stream), n, mats, pivots, info);
-    else
-        hipLaunchKernelGGL(lu_decompose_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), 0,
-                           reinterpret_cast<hipStream_t>(stream), n, mats, pivots, info);
-    RAYSHT_HIP_TRY(hipGetLastError());
-    return RAYSHT_OK;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    // a thread per row; up to 256 rows 512 threads, whose other waves only take trailing tiles, beat
+    // 256 at n = 256 (0.87 against 0.93 ms) and are even at 192
+    if (n <= 64) return launch_lu_decompose<64>(n, nbatch, mats, pivots, info, st);
+    if (n <= 128) return launch_lu_decompose<128>(n, nbatch, mats, pivots, info, st);
+    if (n <= 512) return launch_lu_decompose<512>(n, nbatch, mats, pivots, info, st);
+    return launch_lu_decompose<1024>(n, nbatch, mats, pivots, info, st);
 }
 
 int raysht_lu_solve_full(int n, int nbatch, const double *mats, const int *pivots, double *rhs, const long *rhs_off,
