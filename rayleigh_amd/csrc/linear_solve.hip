@@ -68,11 +68,9 @@ inline bool solve_grid_fits(int ncb, int nbatch, int grouped, int threads)
 // reciprocal, about a third of n = 256), then the passes over the trailing block, which the
 // caches and FP64 vector arithmetic share (matrix instructions would fuse the product into the
 // sum).  256 matrices of n = 64, 128, 256: 0.13, 0.33, 0.87 ms; 128 of n = 512: 3.3 ms, 32 of
-// n = 1000: 19 ms; steps
-// that go through global memory (the search, the interchange of the whole row, the update of
-// the panel) took 0.31, 0.67, 2.39, 9.1 and
-// 45 ms.  Panels of 32 need a step code of 137 KB, more than the
-// instruction cache, and were slower at every n.
+// n = 1000: 19 ms.  Steps that go through global memory (the search, the interchange of the
+// whole row, the update of the panel) took 0.31, 0.67, 2.39, 9.1 and 45 ms.  Panels of 32 need a
+// step code of 137 KB, more than the instruction cache, and were slower at every n.
 constexpr int kLuNB = 16;
 constexpr int kLuChunk = 256;  // rows of L21 and columns of U12 in LDS at a time
 
@@ -353,9 +351,16 @@ int launch_lu_decompose(int n, int nbatch, double *mats, int *pivots, int *info,
 // Solve with the right-hand sides in registers: G lanes of a wave own CPL columns, lane
 // r holds rows r, r + G, ... (NT of them) of each.  The interchanges are composed into one
 // permutation applied when the column is loaded; then each step j takes x_j from its
-// owner lane by a lane shuffle and updates the lane's rows in registers, while the next
-// column of L (or U) is loaded -- no barrier after the permutation.  Operation order and
-// rounding are those of the reference BLAS order.
+// owner lane by a lane shuffle and updates the lane's rows in registers.  The factor comes
+// through LDS K columns at a time, shared by all the workgroup's right-hand sides, the next K on
+// their way in registers meanwhile; one barrier per K columns.  Operation order and rounding are
+// those of the reference BLAS order.
+// With one column on its way per wave the steps waited for memory (each takes a new cache line from
+// every row block) and for the vector cache, which served every wave by itself; rows that a step does not
+// touch were loaded and computed too.  256 matrices of n = 64, 128, 256 with 2 (l + 1) columns
+// each: 0.15, 0.45, 1.33 ms before, 0.14, 0.32, 0.87 ms now (the arithmetic alone takes 0.25 ms of the
+// last); 128 of n = 512 1.64 -> 1.26 ms, 32 of n = 1000 1.48 -> 1.08 ms.  What is left is the chain of a
+// step: a shuffle, LDS reads, a product and a difference.
 template <int G, int NT, int CPL>
 __global__ __launch_bounds__(kLuThreads) void lu_solve_lanes_kernel(int n, int nbatch, int ncb, int grouped,
                                                                     const double *__restrict__ mats,
@@ -365,29 +370,30 @@ __global__ __launch_bounds__(kLuThreads) void lu_solve_lanes_kernel(int n, int n
                                                                     const int *__restrict__ nrhs)
 {
 #pragma clang fp contract(off)
-    __shared__ int perm[G * NT];
+    constexpr int R = G * NT, K = R > 256 ? 4 : 8, PT = K * R / kLuThreads;
+    __shared__ int perm[R];
+    __shared__ double s_col[2 * K * R];
     constexpr int kCols = kLuThreads / G * CPL;
     const solve_block sb = solve_block_of(ncb, nbatch, grouped);
     if (sb.b >= nbatch) return;
     const int b = sb.b, ncol = nrhs[b], col0 = sb.cb * kCols;
     if (col0 >= ncol) return;  // uniform: the whole workgroup leaves
     const double *a = mats + (long)b * n * n;
-    const int *piv = pivots + (long)b * n;
+    const auto piv = (const __attribute__((address_space(4))) int *)(pivots + (long)b * n);  // scalar loads
     const int tid = threadIdx.x;
-    if (tid == 0) {
-        for (int i = 0; i < n; ++i) perm[i] = i;
+    // each thread follows its rows through the interchanges
+    for (int i = tid; i < n; i += kLuThreads) {
+        int pos = i;
+#pragma unroll 8
         for (int k = 0; k < n; ++k) {
             const int p = piv[k] - 1;
-            if (p != k && p >= 0 && p < n) {
-                const int t = perm[k];
-                perm[k] = perm[p];
-                perm[p] = t;
-            }
+            if (p >= 0 && p < n) pos = pos == k ? p : pos == p ? k : pos;
         }
+        perm[pos] = i;
     }
     __syncthreads();
     const int lane = tid % G, cg = col0 + (tid / G) * CPL;
-    double x[CPL][NT], cur[NT], nxt[NT];
+    double x[CPL][NT];
 #pragma unroll
     for (int q = 0; q < CPL; ++q) {
         const bool live = cg + q < ncol;
@@ -398,58 +404,88 @@ __global__ __launch_bounds__(kLuThreads) void lu_solve_lanes_kernel(int n, int n
             x[q][t] = live && i < n ? xg[perm[i]] : 0.0;
         }
     }
-    auto column = [&](int j, double(&v)[NT]) {
+    // Groups of K columns, 0 .. ng - 1 for the lower sweep and back for the upper one.  A buffer of
+    // the matrix's size keeps the reads inside it; rows past the matrix reach no result.
+    const int ng = (n + K - 1) / K;
+    const __amdgpu_buffer_rsrc_t ra =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(a), (short)0, 8 * n * n, 0x00020000);
+    double pf[PT];
+    auto fetch = [&](int s) {
+        const int j0 = K * (s < ng ? s : 2 * ng - 1 - s);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int i = G * t + lane;
-            v[t] = i < n ? a[i + (long)j * n] : 0.0;
+        for (int q = 0; q < PT; ++q) {
+            const int e = tid + q * kLuThreads, off = 8 * ((j0 + e / R) * n + e % R);
+            pf[q] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ra, off, 0, 0));
         }
     };
+    auto stage = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < PT; ++q) s_col[(s & 1) * K * R + tid + q * kLuThreads] = pf[q];
+    };
+    // f(kq) for the columns of a group, the next group on its way meanwhile
+    auto group = [&](int s, auto &&steps) {
+        __syncthreads();
+        if (s + 1 < 2 * ng) fetch(s + 1);
+        steps(s_col + (s & 1) * K * R);
+        if (s + 1 < 2 * ng) stage(s + 1);
+    };
+    fetch(0);
+    stage(0);
     // unit lower: x_i -= x_j l_ij for i > j
-    column(0, cur);
+    static_steps<0, NT>([&](auto block) {
+        constexpr int tb = decltype(block)::value;
+        for (int h = 0; h < G / K; ++h) {
+            const int j0 = G * tb + K * h;
+            if (j0 >= n) break;
+            group(j0 / K, [&](const double *col) {
+#pragma unroll 1
+                for (int kq = 0; kq < K; ++kq) {
+                    const int r = K * h + kq;
+                    double l[NT];
 #pragma unroll
-    for (int tb = 0; tb < NT; ++tb) {
-        for (int r = 0; r < G; ++r) {
-            const int j = G * tb + r;
-            if (j >= n - 1) break;
-            column(j + 1, nxt);
+                    for (int t = tb; t < NT; ++t) l[t] = col[kq * R + G * t + lane];
 #pragma unroll
-            for (int q = 0; q < CPL; ++q) {
-                const double xj = __shfl(x[q][tb], r, G);
-                if (xj != 0.0) {
+                    for (int q = 0; q < CPL; ++q) {
+                        const double xj = __shfl(x[q][tb], r, G);
+                        if (xj != 0.0) {
+                            if (lane > r) x[q][tb] = x[q][tb] - xj * l[tb];
 #pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        if (G * t + lane > j) x[q][t] = x[q][t] - xj * cur[t];
+                            for (int t = tb + 1; t < NT; ++t) x[q][t] = x[q][t] - xj * l[t];
+                        }
+                    }
                 }
-            }
-#pragma unroll
-            for (int t = 0; t < NT; ++t) cur[t] = nxt[t];
+            });
         }
-    }
+    });
     // upper: x_j /= u_jj, then x_i -= x_j u_ij for i < j; x_j is final
-    column(n - 1, cur);
+    static_steps<0, NT>([&](auto block) {
+        constexpr int tb = NT - 1 - decltype(block)::value;
+        for (int h = G / K - 1; h >= 0; --h) {
+            const int j0 = G * tb + K * h;
+            if (j0 >= n) continue;
+            group(2 * ng - 1 - j0 / K, [&](const double *col) {
+#pragma unroll 1
+                for (int kq = min(K, n - j0) - 1; kq >= 0; --kq) {
+                    const int r = K * h + kq;
+                    double u[NT];
 #pragma unroll
-    for (int tb = NT - 1; tb >= 0; --tb) {
-        for (int r = G - 1; r >= 0; --r) {
-            const int j = G * tb + r;
-            if (j >= n) continue;
-            if (j > 0) column(j - 1, nxt);
-            const double ujj = __shfl(cur[tb], r, G);
+                    for (int t = 0; t <= tb; ++t) u[t] = col[kq * R + G * t + lane];
+                    const double ujj = col[kq * R + j0 + kq];
 #pragma unroll
-            for (int q = 0; q < CPL; ++q) {
-                double xj = __shfl(x[q][tb], r, G);
-                if (xj != 0.0) {
-                    xj = xj / ujj;
+                    for (int q = 0; q < CPL; ++q) {
+                        double xj = __shfl(x[q][tb], r, G);
+                        if (xj != 0.0) {
+                            xj = xj / ujj;
+                            if (lane < r) x[q][tb] = x[q][tb] - xj * u[tb];
 #pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        if (G * t + lane < j) x[q][t] = x[q][t] - xj * cur[t];
+                            for (int t = 0; t < tb; ++t) x[q][t] = x[q][t] - xj * u[t];
+                        }
+                        if (lane == r) x[q][tb] = xj;
+                    }
                 }
-                if (lane == r) x[q][tb] = xj;
-            }
-#pragma unroll
-            for (int t = 0; t < NT; ++t) cur[t] = nxt[t];
+            });
         }
-    }
+    });
 #pragma unroll
     for (int q = 0; q < CPL; ++q)
         if (cg + q < ncol) {
@@ -462,8 +498,8 @@ __global__ __launch_bounds__(kLuThreads) void lu_solve_lanes_kernel(int n, int n
         }
 }
 
-// CPL right-hand sides per lane group share every loaded column of the factor (measured:
-// 2 for 16-lane groups, 3 for 32- and 64-lane groups, within the register budget)
+// Two right-hand sides per lane group: three waves per SIMD.  One costs 1.03 ms instead of 0.87 at
+// n = 256 (twice the LDS reads), three 1.07 and four 1.01 (fewer waves).
 template <int G, int NT, int CPL>
 int launch_lanes(int n, int nbatch, const double *mats, const int *pivots, double *rhs, const long *rhs_off,
                  const int *nrhs, int max_nrhs, hipStream_t st)
@@ -945,9 +981,13 @@ int raysht_lu_solve_full(int n, int nbatch, const double *mats, const int *pivot
     else if (n <= 256)
         rc = launch_lanes<16, 16, 2>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
     else if (n <= 512)
-        rc = launch_lanes<32, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
+        rc = launch_lanes<32, 16, 2>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
     else
-        rc = launch_lanes<64, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
+        rc = launch_lanes<64, 16, 2>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
+    // a grid beyond the launch limit: fewer workgroups with three columns each
+    if (rc == RAYSHT_EUNSUPPORTED && n > 256)
+        rc = n <= 512 ? launch_lanes<32, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st)
+                      : launch_lanes<64, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
     if (rc != RAYSHT_OK) return rc;
     RAYSHT_HIP_TRY(hipGetLastError());
     return RAYSHT_OK;

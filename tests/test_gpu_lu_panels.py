@@ -1,4 +1,4 @@
-"""The panelled LU factorisation bit for bit against the oracle at the edges of its panels (16
+"""The panelled LU factorisation and the solve bit for bit against the oracle at the edges of its panels (16
 columns), waves, workgroups and trailing tiles, on matrices whose columns hold what the pivot
 search and the updates treat specially: equal candidates, zero rows of U, zero columns, NaNs and
 infinities."""
@@ -51,3 +51,39 @@ def test_factors_match_the_oracle(ra, n):
             lu, p, inf = O.lu_decompose(m)
         assert np.array_equal(piv_g[b], p) and info_g[b] == inf, (n, b)
         assert np.array_equal(got[b].T, lu, equal_nan=True), (n, b)
+
+
+@pytest.mark.parametrize("n", [1, 3, 7, 8, 9, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 259, 300,
+                               511, 512, 513, 515, 700, 1024])
+def test_solutions_match_the_oracle(ra, n):
+    """right-hand-side counts around a workgroup's columns, zeros of both signs and zero columns,
+    factors with entries that a row past the matrix must not see (infinities, NaN)"""
+    import torch
+    rng = np.random.default_rng(n)
+    nb = 3 if n <= 300 else 2
+    facs, pivs = [], []
+    for b in range(nb):
+        f = rng.standard_normal((n, n)) / n + np.eye(n)
+        if b == 1:
+            f[n // 2, n // 3] = np.inf
+            f[n // 4, (2 * n) // 3] = np.nan
+        facs.append(f)
+        pivs.append(np.array([rng.integers(k, n) + 1 for k in range(n)], dtype=np.int32))
+    counts = [33, 17, 1][:nb]
+    offs = np.concatenate([[0], np.cumsum([c * n + 3 for c in counts])]).astype(np.int64)
+    rhs_np = rng.standard_normal(int(offs[-1]))
+    rhs_np[: n] = 0.0
+    rhs_np[n: 2 * n: 2] = -0.0
+    rhs_np[offs[1]: offs[1] + n: 3] = 0.0
+    d = torch.from_numpy(np.concatenate([f.ravel(order="F") for f in facs])).cuda()
+    rhs = torch.from_numpy(rhs_np.copy()).cuda()
+    ra.lu_solve_full(d, torch.from_numpy(np.concatenate(pivs)).cuda(), rhs, torch.from_numpy(offs[:-1]).cuda(),
+                     torch.tensor(counts, dtype=torch.int32).cuda(), n, max(counts))
+    want = rhs_np.copy()
+    for b in range(nb):
+        bb = rhs_np[offs[b]: offs[b] + counts[b] * n].reshape(counts[b], n).T
+        with np.errstate(all="ignore"):
+            want[offs[b]: offs[b] + counts[b] * n] = O.lu_solve(facs[b], pivs[b], bb).T.ravel()
+    got = rhs.cpu().numpy()
+    assert np.array_equal(got, want, equal_nan=True), n
+    assert np.array_equal(np.signbit(got[got == 0.0]), np.signbit(want[want == 0.0]))
