@@ -635,157 +635,148 @@ __global__ __launch_bounds__(kLuThreads) void band_lu_decompose_kernel(int n, in
 
 // The same factorisation with its active window in LDS.  Step j of dgbtf2 reads and writes
 // only matrix rows j .. j + kl and columns j .. j + kv (the pivot search, the interchange
-// over columns j .. ju <= j + kv, the multipliers and the rank-1 update), so that window,
-// (kl + 1) x (kv + 1) values, lives in an LDS ring (matrix row % (kl + 1), column % (kv + 1),
-// column-major) while the factorisation walks down the band: after step j, row j (U) and
-// column j (L) are final and go to the band storage, and step j + 1 brings in row j + kl + 1
-// (plain band entries) and column j + kv + 1 (rows j + 1 .. j + kl: dgbtf2's zeroed fill-in,
-// so zeros are written, not read).  The arithmetic, its order and the pivot choice are the
-// global-memory kernel's, statement for statement, so the factors and pivots are the same
-// doubles; the difference is that the rank-1 updates no longer read and write the band
-// storage through the caches on every step.  Used where the window and the reduction
-// buffers fit one workgroup's LDS.
-__global__ __launch_bounds__(kLuThreads) void band_lu_decompose_lds_kernel(int n, int kl, int ku, int ldab,
-                                                                           double *__restrict__ mats,
-                                                                           int *__restrict__ pivots,
-                                                                           int *__restrict__ infos)
+// over columns j .. ju <= j + kv, the multipliers and the rank-1 update), so that window
+// lives in an LDS ring (matrix row % (kl + 2), column % (kv + 2), column-major, ld apart)
+// while the factorisation walks down the band.  The ring has one row and one column more
+// than the step uses: row j + kl + 1 (plain band entries, loaded before the pivot search) and
+// column j + kv + 1 (rows j + 1 .. j + kl: dgbtf2's zeroed fill-in, so zeros are written, not
+// read) come in for step j + 1 while step j works.  A step has three barriers: every wave
+// finds the pivot by itself; then the interchange writes row j (U, final) and the scaling
+// column j (L, final) to LDS and the band storage in one pass; then the rank-1 update, in
+// which a thread stays on one ring row and keeps its multiplier in a register.  The arithmetic,
+// its order and the pivot choice are the global-memory kernel's, so the factors and pivots
+// are the same doubles.  Used where the window fits one workgroup's LDS.
+// What bounds it is the chain of a column's phases (LDS latency, the barriers), then the LDS
+// rate of the update (three accesses per element).  With seven barriers a step, four LDS accesses per element
+// and 256 threads at every size it took, ms, against now: 170 matrices of n = 192, kl = 72 .813, .420;
+// 128, 40 .377, .186; 64, 20 .167, .080; 256 of n = 256, kl = 96 1.37, .704; n = 512, kl = 8 1.38, .637.
+template <int NT>
+__global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl, int ku, int ldab, int ld,
+                                                                   double *__restrict__ mats,
+                                                                   int *__restrict__ pivots, int *__restrict__ infos)
 {
 #pragma clang fp contract(off)
     extern __shared__ double win[];
-    __shared__ double s_val[kLuThreads];
-    __shared__ int s_idx[kLuThreads];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     double *ab = mats + (long)blockIdx.x * ldab * n;
     int *piv = pivots + (long)blockIdx.x * n;
-    const int kv = ku + kl, R = kl + 1, C = kv + 1;
+    const int kv = ku + kl, R = kl + 2, C = kv + 2;
 #define AB(i, j) ab[(long)((j) - 1) * ldab + ((i) - 1)]
-#define W(row, col) win[((col) % C) * R + ((row) % R)]
-    // the first window, rows 1 .. min(R, n) x columns 1 .. min(C, n); entries more than ku
-    // above the diagonal are fill-in, zero at the start
+    // the first window, rows 1 .. min(kl + 1, n) x columns 1 .. min(kv + 1, n); entries more than
+    // ku above the diagonal are fill-in, zero at the start
     {
-        const int nrw = min(R, n), ncl = min(C, n);
-        for (int e = tid; e < nrw * ncl; e += kLuThreads) {
+        const int nrw = min(kl + 1, n), ncl = min(kv + 1, n);
+        for (int e = tid; e < nrw * ncl; e += NT) {
             const int row = 1 + e % nrw, col = 1 + e / nrw;
-            W(row, col) = col - row > ku ? 0.0 : AB(kv + 1 + row - col, col);
+            win[col * ld + row] = col - row > ku ? 0.0 : AB(kv + 1 + row - col, col);
         }
     }
     __syncthreads();
-    int info = 0, ju = 1;
+    const int rs = tid % ld, g = tid / ld, G = NT / ld;  // the update's ring row and its columns g, g + G, ...
+    int info = 0, ju = 1, jr = 1, jc = 1;                // jr, jc: the ring row and column of j
     for (int j = 1; j <= n; ++j) {
-        if (j > 1) {
-            // row j + kl (columns j .. j + kv) and column j + kv (rows j .. j + kl - 1) into the
-            // slots of row and column j - 1, written out at the end of the previous step
-            const int rn = j + kl, cn = j + kv;
-            if (rn <= n)
-                for (int col = j + tid; col <= min(cn, n); col += kLuThreads) W(rn, col) = AB(kv + 1 + rn - col, col);
-            if (cn <= n)
-                for (int row = j + tid; row <= min(rn - 1, n); row += kLuThreads) W(row, cn) = 0.0;
-            __syncthreads();
-        }
-        const int km = min(kl, n - j);
+        // ring rows / columns at an offset below R / C from j
+        auto ring_row = [&](int i) { return jr + i >= R ? jr + i - R : jr + i; };
+        auto ring_col = [&](int c) { return jc + c >= C ? jc + c - C : jc + c; };
+        const int km = min(kl, n - j), rn = j + kl + 1, cn = j + kv + 1;
+        const double in = rn <= n && j + 1 + tid <= min(cn, n) ? AB(kv + rn - j - tid, j + 1 + tid) : 0.0;
+        double *colj = win + jc * ld;
+        // the largest |a| with the lowest index among equals; NaNs never enter
         double best = -1.0;
         int bi = 1 << 30;
-        for (int i = 1 + tid; i <= km + 1; i += kLuThreads) {
-            const double v = fabs(W(j + i - 1, j));
+        for (int i = lane; i <= km; i += 64) {
+            const double v = fabs(colj[ring_row(i)]);
             if (v > best) {
                 best = v;
                 bi = i;
             }
         }
-        // the largest |a| with the lowest index among equals: a total order on the candidates
-        // (NaNs never enter), so the shuffle and cross-wave order cannot change the choice
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double v = __shfl_xor(best, off);
-            const int q = __shfl_xor(bi, off);
-            if (v > best || (v == best && q < bi)) {
-                best = v;
-                bi = q;
-            }
-        }
-        if ((tid & 63) == 0) {
-            s_val[tid >> 6] = best;
-            s_idx[tid >> 6] = bi;
-        }
-        __syncthreads();
-        best = s_val[0];
-        bi = s_idx[0];
-#pragma unroll
-        for (int w = 1; w < kLuThreads / 64; ++w)
-            if (s_val[w] > best || (s_val[w] == best && s_idx[w] < bi)) {
-                best = s_val[w];
-                bi = s_idx[w];
-            }
+        const double wm = lu_wave_max(best);
+        unsigned long long eq = __ballot(best == wm);
+        int p = __builtin_amdgcn_readlane(bi, __builtin_ctzll(eq));
+        for (eq &= eq - 1; eq != 0; eq &= eq - 1)
+            p = min(p, (int)__builtin_amdgcn_readlane(bi, __builtin_ctzll(eq)));
         // idamax: a NaN first entry is kept (nothing compares larger); later NaNs are passed over
-        const int jp = (bi > km + 1 || isnan(W(j, j))) ? 1 : bi;
-        const double pv = W(j + jp - 1, j);
-        __syncthreads();  // every thread has the pivot before the interchange moves it
-        if (tid == 0) piv[j - 1] = jp + j - 1;
-        if (pv != 0.0) {
-            ju = max(ju, min(j + ku + jp - 1, n));
-            if (jp != 1)
-                for (int c = tid; c <= ju - j; c += kLuThreads) {
-                    const double t = W(j + jp - 1, j + c);
-                    W(j + jp - 1, j + c) = W(j, j + c);
-                    W(j, j + c) = t;
-                }
-            __syncthreads();
-            if (km > 0) {
-                const double r = 1.0 / W(j, j);
-                for (int i = 1 + tid; i <= km; i += kLuThreads) W(j + i, j) = r * W(j + i, j);
-                __syncthreads();
-                // element e = (i - 1) + km (c - 1) of the update, e = tid, tid + kLuThreads, ...:
-                // i, c and their ring slots stepped by kLuThreads elements without divisions
-                const int w = ju - j, di = kLuThreads % km, dc = (kLuThreads / km) % C;
-                int ii = tid % km, rs = (j + 1 + ii) % R, cs = (j + 1 + tid / km) % C;
-                const int js = j % R, jc = (j % C) * R, tot = km * w;
-                // four elements per thread at a time: their operands (row j and column j are
-                // not written by the update) are read before any of the four is written
-                constexpr int U = 4;
-                for (int e = tid; e < tot; e += U * kLuThreads) {
-                    int rsu[U], csu[U];
-                    bool on[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        on[u] = e + u * kLuThreads < tot;
-                        rsu[u] = on[u] ? rs : 0;
-                        csu[u] = on[u] ? cs : 0;
-                        ii += di;
-                        rs += di;
-                        if (rs >= R) rs -= R;
-                        cs += dc;
-                        if (ii >= km) {
-                            ii -= km;
-                            rs -= km;
-                            if (rs < 0) rs += R;
-                            ++cs;
-                        }
-                        if (cs >= C) cs -= C;
-                    }
-                    double y[U], a[U], x[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        y[u] = win[csu[u] * R + js];
-                        a[u] = win[csu[u] * R + rsu[u]];
-                        x[u] = win[jc + rsu[u]];
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (on[u] && y[u] != 0.0) win[csu[u] * R + rsu[u]] = a[u] + x[u] * (-y[u]);
-                }
-                __syncthreads();
-            }
-        } else if (info == 0) {
+        const double d0 = colj[jr];
+        if (p > km || isnan(d0)) p = 0;
+        const int pr = ring_row(p);
+        const double pv = colj[pr];
+        __syncthreads();  // every wave has the pivot before the interchange moves it
+        if (tid == 0) piv[j - 1] = j + p;
+        const bool work = pv != 0.0;
+        if (work)
+            ju = max(ju, min(j + ku + p, n));
+        else if (info == 0)
             info = j;
+        // row j of columns j + 1 .. (the first half of the threads), column j (the second half)
+        const int w = ju - j, ncr = min(kv, n - j);
+        if (tid < NT / 2) {
+            for (int c = 1 + tid; c <= ncr; c += NT / 2) {
+                double *col = win + ring_col(c) * ld;
+                const double old = col[jr];
+                double u = old;
+                if (work && p != 0 && c <= w) {
+                    u = col[pr];
+                    col[pr] = old;
+                    col[jr] = u;
+                }
+                AB(kv + 1 - c, j + c) = u;
+            }
+        } else {
+            const double r = 1.0 / pv;
+            for (int i = tid - NT / 2; i <= km; i += NT / 2) {
+                double l = i == 0 ? pv : i == p ? d0 : colj[ring_row(i)];  // without a pivot p = 0
+                if (work && i > 0) l = r * l;
+                if (i > 0) colj[ring_row(i)] = l;
+                AB(kv + 1 + i, j) = l;
+            }
         }
-        // row j (columns j .. j + kv) and column j (rows j + 1 .. j + kl) are final
-        for (int col = j + tid; col <= min(j + kv, n); col += kLuThreads) AB(kv + 1 + j - col, col) = W(j, col);
-        for (int row = j + 1 + tid; row <= min(j + kl, n); row += kLuThreads) AB(kv + 1 + row - j, j) = W(row, j);
+        // row and column of the next step into the ring slots of row and column j - 1
+        const int nr = jr > 0 ? jr - 1 : R - 1, ncol = jc > 0 ? jc - 1 : C - 1;
+        if (rn <= n)
+            for (int c = tid; c <= min(kv, n - j - 1); c += NT)
+                win[ring_col(c + 1) * ld + nr] = c == tid ? in : AB(kv + rn - j - c, j + 1 + c);
+        if (cn <= n)
+            for (int i = 1 + tid; i <= min(kl, n - j); i += NT) win[ncol * ld + ring_row(i)] = 0.0;
         __syncthreads();
+        int i = rs - jr;
+        if (i < 0) i += R;
+        if (work && rs < R && g < G && i >= 1 && i <= km) {
+            const double x = colj[rs];
+            constexpr int U = 4;
+            int cs = jc + 1 + g;
+            for (int c = 1 + g; c <= w; c += U * G) {
+                double y[U], a[U];
+                int at[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bool on = c + u * G <= w;
+                    if (cs >= C) cs -= C;
+                    at[u] = on ? cs * ld : jc * ld;
+                    cs += G;
+                    y[u] = win[at[u] + jr];
+                    a[u] = win[at[u] + rs];
+                    if (!on) y[u] = 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (y[u] != 0.0) win[at[u] + rs] = a[u] + x * (-y[u]);
+            }
+        }
+        __syncthreads();
+        if (++jr == R) jr = 0;
+        if (++jc == C) jc = 0;
     }
     if (tid == 0) infos[blockIdx.x] = info;
-#undef W
 #undef AB
+}
+
+template <int NT>
+void launch_band_lds(int n, int kl, int ku, int nbatch, double *mats, int ldab, int ld, int *pivots, int *info,
+                     hipStream_t st)
+{
+    hipLaunchKernelGGL((band_lu_decompose_lds_kernel<NT>), dim3((unsigned)nbatch), dim3(NT),
+                       sizeof(double) * (size_t)ld * (kl + ku + 2), st, n, kl, ku, ldab, ld, mats, pivots, info);
 }
 
 // Banded solve: LU_Solve_Band (Linear_Solve.F90:1056-1086, dgbtrs 'N').  One wave solves CPL
@@ -1001,17 +992,26 @@ int raysht_lu_decompose_band(int n, int kl, int ku, int nbatch, double *mats, in
     if (nbatch > 0 && (!mats || !pivots || !info)) return RAYSHT_EINVAL;
     if (kl + ku > kBandMaxKv) return RAYSHT_EUNSUPPORTED;
     if (nbatch == 0) return RAYSHT_OK;
-    // the LDS-window kernel where its window and reduction buffers fit one workgroup's LDS
-    const size_t win = sizeof(double) * (size_t)(kl + 1) * (kl + ku + 1);
+    // the LDS-window kernel where its window fits one workgroup's LDS; an odd distance between columns
+    // keeps the interchange of a row off the same banks
     int dev = 0, lds_max = 0;
     RAYSHT_HIP_TRY(hipGetDevice(&dev));
     RAYSHT_HIP_TRY(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    if (win + kLuThreads * (sizeof(double) + sizeof(int)) <= (size_t)lds_max)
-        hipLaunchKernelGGL(band_lu_decompose_lds_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), win,
-                           reinterpret_cast<hipStream_t>(stream), n, kl, ku, ldab, mats, pivots, info);
+    const size_t cols = sizeof(double) * (size_t)(kl + ku + 2), most = (size_t)lds_max;
+    const int ld = cols * (size_t)((kl + 2) | 1) <= most ? (kl + 2) | 1 : kl + 2;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    // threads by the size of the rank-1 update: 256 / 512 / 1024 take .080 / .089 / .100 ms at n = 64,
+    // kl = 20 (170 matrices), .208 / .186 / .225 at 128, 40, .552 / .420 / .433 at 192, 72 and
+    // 1.196 / .726 / .704 at 256, 96 (256 matrices)
+    if (cols * ld <= most && kl <= 24)
+        launch_band_lds<256>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (cols * ld <= most && kl <= 80)
+        launch_band_lds<512>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (cols * ld <= most)
+        launch_band_lds<1024>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
     else
-        hipLaunchKernelGGL(band_lu_decompose_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), 0,
-                           reinterpret_cast<hipStream_t>(stream), n, kl, ku, ldab, mats, pivots, info);
+        hipLaunchKernelGGL(band_lu_decompose_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), 0, st, n, kl,
+                           ku, ldab, mats, pivots, info);
     RAYSHT_HIP_TRY(hipGetLastError());
     return RAYSHT_OK;
 }
