@@ -791,6 +791,16 @@ void launch_band_lds(int n, int kl, int ku, int nbatch, double *mats, int ldab, 
 // in the loop bodies is a compile-time register index (a select over NS slots per access
 // was most of the kernel's instructions).  Segments advance by one rotation of the NS
 // slots, and NS rotations restore the natural order.
+// What bounds it is the chain of a step: the factor column's load (asked for before anything
+// else of the step), x_j, the division.  x_j and the interchange's rows are read with v_readlane, a
+// segment's pivots are held one per lane, and one division serves the CPL columns, lane c
+// dividing for column c.  With LDS-path shuffles, a pivot load per step and a division per column it took, ms,
+// against now: 256 matrices of n = 256, kl = 96 2.18, 1.75; 170 of n = 192, kl = 72 .734, .632; 64, 20
+// .222, .203; 64 of n = 300, kl = 98 .759, .711; 64 of n = 600, kl = 40 1.79, 1.69; 256 of n = 512, kl = 8 is
+// even at 4.4.  The next step's column loaded one to four steps ahead costs registers and so
+// waves: 2.54 instead of 1.75 ms at n = 256.  Slots outside the band are passed over in the load for
+// NS >= 8 only (NS = 4: 1.98 ms at n = 256 with that branch), and NS = 8 is held to four waves per SIMD (4.4
+// against 5.0 ms at n = 512, kl = 8).
 template <int NS>
 __device__ __forceinline__ void slots_rotate_down(double (&x)[NS])  // slot k takes slot k + 1
 {
@@ -809,27 +819,16 @@ __device__ __forceinline__ void slots_rotate_up(double (&x)[NS])  // slot k take
     x[0] = xl;
 }
 
-// value of row `row`, in relative slot (row >> 6) - S (0 .. NS - 1 - S)
-template <int NS>
-__device__ __forceinline__ double band_row(const double (&x)[NS], int rel, int row)
+// the value of lane `l` (the same in every lane)
+__device__ __forceinline__ double lane_value(double v, int l)
 {
-    double v = x[0];
-#pragma unroll
-    for (int k = 1; k < NS; ++k)
-        if (k == rel) v = x[k];
-    return __shfl(v, row & 63);
-}
-
-template <int NS>
-__device__ __forceinline__ void band_set(double (&x)[NS], int rel, int row, int lane, double v)
-{
-#pragma unroll
-    for (int k = 0; k < NS; ++k)
-        if (k == rel && lane == (row & 63)) x[k] = v;
+    const long b = __builtin_bit_cast(long, v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __builtin_bit_cast(double, ((long)hi << 32) | (unsigned)lo);
 }
 
 template <int NS, int CPL>
-__global__ __launch_bounds__(64) void band_lu_solve_kernel(int n, int kl, int ku, int ldab, int nbatch, int ncb,
+__global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int n, int kl, int ku, int ldab, int nbatch, int ncb,
                                                            const double *__restrict__ mats,
                                                            const int *__restrict__ pivots, double *__restrict__ rhs,
                                                            const long *__restrict__ rhs_off,
@@ -853,34 +852,63 @@ __global__ __launch_bounds__(64) void band_lu_solve_kernel(int n, int kl, int ku
             const int r = s * 64 + lane;
             x[c][s] = (c < nc && r < n) ? x0[(long)c * n + r] : 0.0;
         }
+    constexpr int D = NS == 1 ? 2 : 1;  // steps whose factor columns are loaded together
     // L solve with the interchanges, segment by segment (row j in slot 0)
 #pragma unroll 1
     for (int S = 0; S < NS; ++S) {
         const int jend = kl > 0 ? min(64 * (S + 1), n - 1) : 0;
-        for (int j = 64 * S; j < jend; ++j) {
-            const int jj = j & 63, lm = min(kl, n - 1 - j), l = piv[j] - 1, lrel = (l >> 6) - S;
-            double y[CPL];
+        const int pj = 64 * S + lane < n ? piv[64 * S + lane] : 0;
+        double a[D][NS];
+        auto fetch = [&](int j0) {
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                if (l != j) {
-                    const double xl = band_row(x[c], lrel, l), xj = __shfl(x[c][0], jj);
-                    if (lane == jj) x[c][0] = xl;
-                    band_set(x[c], lrel, l, lane, xj);
+            for (int d = 0; d < D; ++d) {
+                const int j = j0 + d, lm = min(kl, n - 1 - j);
+                const double *col = ab + (long)j * ldab + kv - j;  // col[r] = factor entry (r, j)
+#pragma unroll
+                for (int k = 0; k < NS; ++k) {
+                    const int r = (S + k) * 64 + lane;
+                    if (NS >= 8 && ((S + k) * 64 + 63 <= j || (S + k) * 64 > j + lm)) continue;
+                    a[d][k] = j < jend && r > j && r <= j + lm ? col[r] : 0.0;
                 }
-                y[c] = __shfl(x[c][0], jj);
             }
-            const int klo = ((j + 1) >> 6) - S, khi = ((j + lm) >> 6) - S;
-            const double *col = ab + (long)j * ldab + kv - j;  // col[r] = factor entry (r, j)
+        };
+#pragma unroll 1
+        for (int j0 = 64 * S; j0 < jend; j0 += D) {
+            fetch(j0);
+            static_steps<0, D>([&](auto step) {
+#pragma clang fp contract(off)
+                constexpr int d = decltype(step)::value;
+                const int j = j0 + d;
+                if (j >= jend) return;
+                const int jj = j & 63, lm = min(kl, n - 1 - j);
+                const int l = __builtin_amdgcn_readlane(pj, jj) - 1, lrel = (l >> 6) - S;
+                double y[CPL];
 #pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                if (k < klo || k > khi) continue;
-                const int r = (S + k) * 64 + lane;
-                if (r <= j || r > j + lm) continue;
-                const double a = col[r];
+                for (int c = 0; c < CPL; ++c) y[c] = lane_value(x[c][0], jj);
+                if (l != j)
+                    static_steps<0, NS>([&](auto slot) {
+                        constexpr int k = decltype(slot)::value;
+                        if (k != lrel) return;
+                        asm volatile("" ::"n"(k));  // keeps the slots' branches apart: x[lrel] would put x into memory
 #pragma unroll
-                for (int c = 0; c < CPL; ++c)
-                    if (y[c] != 0.0) x[c][k] = x[c][k] + a * (-y[c]);
-            }
+                        for (int c = 0; c < CPL; ++c) {
+                            const double xl = lane_value(x[c][k], l & 63);
+                            if (lane == jj) x[c][0] = xl;
+                            if (lane == (l & 63)) x[c][k] = y[c];
+                            y[c] = xl;
+                        }
+                    });
+                const int klo = ((j + 1) >> 6) - S, khi = ((j + lm) >> 6) - S;
+#pragma unroll
+                for (int k = 0; k < NS; ++k) {
+                    if (k < klo || k > khi) continue;
+                    const int r = (S + k) * 64 + lane;
+                    if (r <= j || r > j + lm) continue;
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c)
+                        if (y[c] != 0.0) x[c][k] = x[c][k] + a[d][k] * (-y[c]);
+                }
+            });
         }
 #pragma unroll
         for (int c = 0; c < CPL; ++c) slots_rotate_down(x[c]);
@@ -890,34 +918,62 @@ __global__ __launch_bounds__(64) void band_lu_solve_kernel(int n, int kl, int ku
     for (int S = NS - 1; S >= 0; --S) {
 #pragma unroll
         for (int c = 0; c < CPL; ++c) slots_rotate_up(x[c]);
-        for (int j = min(64 * S + 63, n - 1); j >= 64 * S; --j) {
-            const int jj = j & 63;
-            const double *col = ab + (long)j * ldab + kv - j;
-            const double d = col[j];
-            double t[CPL];
-            bool nz[CPL];  // dtbsv skips a column where x(j) is 0 before the division
+        double a[D][NS], dg[D];
+        auto fetch = [&](int j0) {
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                t[c] = __shfl(x[c][0], jj);
-                nz[c] = t[c] != 0.0;
-                if (nz[c]) {
-                    t[c] = t[c] / d;
-                    if (lane == jj) x[c][0] = t[c];
+            for (int d = 0; d < D; ++d) {
+                const int j = j0 - d, lo = max(0, j - kv);
+                const bool on = j >= 64 * S;
+                const double *col = ab + (long)j * ldab + kv - j;
+                dg[d] = on ? col[j] : 1.0;
+#pragma unroll
+                for (int k = 0; k < NS; ++k) {
+                    const int sa = k == 0 ? S : S - (NS - k);  // absolute slot of relative slot k
+                    const int r = sa * 64 + lane;
+                    if (NS >= 8 && (sa * 64 + 63 < lo || sa * 64 >= j)) continue;
+                    a[d][k] = on && r >= lo && r < j ? col[r] : 0.0;
                 }
             }
-            if (j == 0) continue;
-            const int lo = max(0, j - kv), slo = lo >> 6, shi = (j - 1) >> 6;
+        };
+        const int jtop = min(64 * S + 63, n - 1);
+#pragma unroll 1
+        for (int j0 = jtop; j0 >= 64 * S; j0 -= D) {
+            fetch(j0);
+            static_steps<0, D>([&](auto step) {
+#pragma clang fp contract(off)
+                constexpr int d = decltype(step)::value;
+                const int j = j0 - d;
+                if (j < 64 * S) return;
+                const int jj = j & 63;
+                // lane c divides for column c; dtbsv skips a column where x(j) is 0 before the division
+                double t[CPL], q = 0.0;
+                bool nz[CPL];
 #pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                const int sa = k == 0 ? S : S - (NS - k);  // absolute slot of relative slot k
-                if (sa < slo || sa > shi) continue;
-                const int r = sa * 64 + lane;
-                if (r < lo || r >= j) continue;
-                const double a = col[r];
+                for (int c = 0; c < CPL; ++c) {
+                    t[c] = lane_value(x[c][0], jj);
+                    nz[c] = t[c] != 0.0;
+                    if (lane == c) q = t[c];
+                }
+                q = q / dg[d];
 #pragma unroll
                 for (int c = 0; c < CPL; ++c)
-                    if (nz[c]) x[c][k] = x[c][k] - t[c] * a;
-            }
+                    if (nz[c]) {
+                        t[c] = lane_value(q, c);
+                        if (lane == jj) x[c][0] = t[c];
+                    }
+                if (j == 0) return;
+                const int lo = max(0, j - kv), slo = lo >> 6, shi = (j - 1) >> 6;
+#pragma unroll
+                for (int k = 0; k < NS; ++k) {
+                    const int sa = k == 0 ? S : S - (NS - k);
+                    if (sa < slo || sa > shi) continue;
+                    const int r = sa * 64 + lane;
+                    if (r < lo || r >= j) continue;
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c)
+                        if (nz[c]) x[c][k] = x[c][k] - t[c] * a[d][k];
+                }
+            });
         }
     }
 #pragma unroll

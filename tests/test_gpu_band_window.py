@@ -1,4 +1,4 @@
-"""The banded LU factorisation with its window in LDS bit for bit against the oracle: window
+"""The banded LU factorisation with its window in LDS, and the solve, bit for bit against the oracle: window
 sizes around a wave and around the largest that fits (kl = ku = 99 is the last), matrices
 smaller than their window, unequal bands, and columns that the pivot search and the updates
 treat specially (equal candidates, zero columns, zeros in the pivot row, NaN, infinities)."""
@@ -53,3 +53,38 @@ def test_factors_match_the_oracle(n, kl, ku):
         assert np.array_equal(piv_g[b], p) and info_g[b] == inf, (n, kl, ku, b)
         assert np.array_equal(got[b].T, f, equal_nan=True), (n, kl, ku, b)
         assert np.array_equal(np.signbit(got[b].T[f == 0.0]), np.signbit(f[f == 0.0])), (n, kl, ku, b)
+
+
+@pytest.mark.parametrize("n,kl,ku", [(1, 0, 0), (2, 1, 1), (63, 62, 62), (64, 3, 3), (65, 64, 64), (128, 70, 70),
+                                     (129, 5, 9), (192, 72, 72), (255, 130, 2), (257, 96, 96), (512, 8, 8),
+                                     (513, 70, 3), (1000, 65, 65), (1024, 2, 130)])
+def test_solutions_match_the_oracle(n, kl, ku):
+    """column counts around a wave's columns, zeros of both signs, whole zero columns, an infinity"""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import rayleigh_amd as ra
+    rng = np.random.default_rng(n + kl)
+    facs, pivs, counts = [], [], [11, 4, 1]
+    for m in matrices(n, kl, ku)[:2] + matrices(n, kl, ku)[:1]:
+        with np.errstate(all="ignore"):
+            f, p, _ = O.band_lu_decompose(ra.band_storage(m, kl, ku), kl, ku)
+        facs.append(f)
+        pivs.append(p)
+    offs = np.concatenate([[0], np.cumsum([c * n + 3 for c in counts])]).astype(np.int64)
+    rhs_np = rng.standard_normal(int(offs[-1]))
+    rhs_np[: n] = 0.0
+    rhs_np[n: 2 * n: 2] = -0.0
+    rhs_np[2 * n + n // 2] = np.inf
+    rhs_np[offs[2]: offs[2] + n: 3] = 0.0
+    rhs = torch.from_numpy(rhs_np.copy()).cuda()
+    ra.lu_solve_band(torch.from_numpy(np.concatenate([f.ravel(order="F") for f in facs])).cuda(),
+                     torch.from_numpy(np.concatenate(pivs)).cuda(), rhs, torch.from_numpy(offs[:-1]).cuda(),
+                     torch.tensor(counts, dtype=torch.int32).cuda(), n, kl, max(counts), ku=ku)
+    got, want = rhs.cpu().numpy(), rhs_np.copy()
+    for b, c in enumerate(counts):
+        bb = rhs_np[offs[b]: offs[b] + c * n].reshape(c, n).T
+        with np.errstate(all="ignore"):
+            want[offs[b]: offs[b] + c * n] = O.band_lu_solve(facs[b], kl, ku, pivs[b], bb).T.ravel()
+    assert np.array_equal(got, want, equal_nan=True), (n, kl, ku)
+    assert np.array_equal(np.signbit(got[got == 0.0]), np.signbit(want[want == 0.0])), (n, kl, ku)
