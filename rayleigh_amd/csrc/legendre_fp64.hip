@@ -100,7 +100,7 @@ static_assert(STP_KC * STP_TJ == 2 * STP_THREADS, "one 16-byte table piece per t
 // One workgroup per work item; the hardware dispatcher balances the uneven items
 // (a persistent variant that prefetched across items measured slower).
 struct stp_item {
-    int j0, c0, nl, ne, no;
+    int j0, c0, nl, ne, no, nt_stores;
     __amdgpu_buffer_rsrc_t rs, rpe, rpo, ro;
 };
 
@@ -201,20 +201,22 @@ __device__ __forceinline__ void stp_tile(const stp_item &cur, int nt, int nt2, i
                 step(T, s, l + 8 * s < cur.nl ? d[s].x : 0.0, l + 8 * s + 1 < cur.nl ? d[s].y : 0.0);
     }
     // Rows past nrhs lie past the buffer and are dropped; nodes past the equator (the last
-    // block only) are skipped.  Non-temporal: nothing reads the output before this launch
-    // ends, and it would push the tables and input columns that other tiles share out of L2
-    // (l_max = 169, N_r = 96, 6 fields: StP 0.137 -> 0.115 ms).
+    // block only) are skipped.
     const int vn = ((wc + lg) * nt + cur.j0 + li) * 8;                            // + 128 b
     const int vs = ((wc + lg) * nt + nt - 1 - cur.j0 - li - 16 * (NB - 1)) * 8;  // + 128 (NB - 1 - b)
+    auto store = [&](auto put) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+        for (int v = 0; v < 4; ++v)
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-            if (b < NB - 1 || cur.j0 + 16 * b + li < nt2) {
-                const double e = acc_e[b][v], o = acc_o[b][v];
-                store_f64_nt(cur.ro, vn + v * nt * 32 + 128 * b, e + o);
-                store_f64_nt(cur.ro, vs + v * nt * 32 + 128 * (NB - 1 - b), e - o);
-            }
+            for (int b = 0; b < NB; ++b)
+                if (b < NB - 1 || cur.j0 + 16 * b + li < nt2) {
+                    const double e = acc_e[b][v], o = acc_o[b][v];
+                    put(cur.ro, vn + v * nt * 32 + 128 * b, e + o);
+                    put(cur.ro, vs + v * nt * 32 + 128 * (NB - 1 - b), e - o);
+                }
+    };
+    if (cur.nt_stores) store(store_f64_nt);
+    else store(store_f64);
 }
 
 __global__ __launch_bounds__(STP_THREADS, kFp64MinWaves) void stp_fp64_kernel(
@@ -229,6 +231,7 @@ __global__ __launch_bounds__(STP_THREADS, kFp64MinWaves) void stp_fp64_kernel(
     const int nt2 = uniform(it.nt2), nrhs = uniform(it.nrhs), pi = uniform(it.prob), nb = uniform(it.blocks);
     cur.j0 = uniform(it.r0);
     cur.c0 = uniform(it.c0);
+    cur.nt_stores = uniform(it.nt_stores);
     cur.ne = (cur.nl + 1) >> 1;
     cur.no = cur.nl >> 1;
     cur.rs = make_rsrc(uniform(io.in[pi]) + uniform(it.s_off), (long)cur.nl * nrhs * 8);

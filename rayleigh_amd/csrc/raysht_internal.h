@@ -50,7 +50,7 @@ struct fp64_item {
     int nt2, nrhs;          // N_theta / 2, columns
     int prob;               // problem index: which input and output of the launch
     int blocks;             // 16-row blocks of the tile, 1 .. 4
-    int pad;
+    int nt_stores;          // StP: the output is stored past the caches
 };
 static_assert(sizeof(fp64_item) == 64, "one cache line half per item");
 

@@ -55,6 +55,24 @@ void device_free(T *&ptr)
 int n_even(int lmax, int m) { return (lmax - m + 2) / 2; }
 int n_odd(int lmax, int m) { return (lmax - m + 1) / 2; }
 
+// StP stores past the caches (non-temporal) where the 16 nodes of a store are a whole 128-byte
+// line, N_theta a multiple of 16: nothing reads the output before the launch ends, and it would
+// push the tables and input columns that other tiles share out of L2 (l_max = 169, N_theta =
+// 256, N_r = 96, 3 fields: 74 us through the caches, 62 past them).  Elsewhere a store leaves
+// parts of lines.  Past the caches these merge only where the output is small: l_max = 83,
+// N_theta = 126 takes 11.8 us through the caches and 10.9 past them with 22 MB of output (N_r =
+// 64, 2 fields), 17 and 23 with 49 MB, 24 and 42 with 87 MB, and l_max = 179, N_theta = 270 171 and
+// 191 with 398 MB.  Half lines (N_theta a multiple of 8): 39 MB 16.0 / 14.2 us, 66 MB 34.7 / 32.8,
+// 86 MB 26.4 / 29.2, 154 MB 44 / 50, and the other way round once the output no longer leaves the
+// last-level cache (256 MB) room for anything else: 218 MB 81 / 71, 308 MB 111 / 91.
+bool stores_past_caches(const raysht_plan *p)
+{
+    const double bytes = 8.0 * p->nt * p->nrhs * p->nm;
+    if (p->nt % 16 == 0) return true;
+    if (p->nt % 8 == 0) return bytes <= 70e6 || bytes >= 192e6;
+    return bytes <= 32e6;
+}
+
 }  // namespace
 
 // The FP64 kernels' work list.  Inside an m-block the row tiles of one column tile are
@@ -100,6 +118,7 @@ std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, 
         it.nt2 = p->nt2;
         it.nrhs = p->nrhs;
         it.prob = b.prob;
+        it.nt_stores = stp && stores_past_caches(p);
         std::vector<fp64_item> items;
         // column tile outer, row tile inner: consecutive items share the column tile's
         // input (spectral columns for StP, hybrid columns for PtS) while it is in L2
