@@ -106,6 +106,16 @@ __device__ __forceinline__ void static_steps(F &&f)
     }
 }
 
+// the same until f returns false
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_while(F &&f)
+{
+    if constexpr (I < N) {
+        if (!f(std::integral_constant<int, I>{})) return;
+        static_while<I + 1, N>(f);
+    }
+}
+
 // LDS of one workgroup: two sets of candidate rows, L11, the moves, U12 and L21 chunks
 __host__ __device__ inline int lu_chunk(int n) { return n < kLuChunk ? n : kLuChunk; }
 __host__ __device__ inline int lu_ld(int n) { return lu_chunk(n) | 1; }
@@ -798,9 +808,14 @@ void launch_band_lds(int n, int kl, int ku, int nbatch, double *mats, int ldab, 
 // against now: 256 matrices of n = 256, kl = 96 2.18, 1.75; 170 of n = 192, kl = 72 .734, .632; 64, 20
 // .222, .203; 64 of n = 300, kl = 98 .759, .711; 64 of n = 600, kl = 40 1.79, 1.69; 256 of n = 512, kl = 8 is
 // even at 4.4.  The next step's column loaded one to four steps ahead costs registers and so
-// waves: 2.54 instead of 1.75 ms at n = 256.  Slots outside the band are passed over in the load for
-// NS >= 8 only (NS = 4: 1.98 ms at n = 256 with that branch), and NS = 8 is held to four waves per SIMD (4.4
-// against 5.0 ms at n = 512, kl = 8).
+// waves: 2.54 instead of 1.75 ms at n = 256.  NS = 8 is held to four waves per SIMD (4.4 against 5.0 ms at
+// n = 512, kl = 8).
+// For NS >= 4 a pass over the slots leaves where the band ends, so a step costs what its band
+// reaches: the slots of a step are neighbours (downwards from row j's in the L solve, upwards in the
+// U solve).  A branch around each of the 16 or 32 slots outside the band, in the load and again in the
+// update, was most of a narrow band's step; ms with those branches, now, 170 matrices with 2 (l + 1)
+// columns: n = 192, kl = 72 .626, .585; 256, 96 .877, .843; 300, 98 1.76, 1.19; 512, 8 2.21, 1.40;
+// 600, 40 7.79, 5.31; 1000, 4 11.8, 6.5.  NS = 1 and 2 are even (one branch, at most two slots).
 template <int NS>
 __device__ __forceinline__ void slots_rotate_down(double (&x)[NS])  // slot k takes slot k + 1
 {
@@ -817,6 +832,18 @@ __device__ __forceinline__ void slots_rotate_up(double (&x)[NS])  // slot k take
 #pragma unroll
     for (int k = NS - 1; k > 0; --k) x[k] = x[k - 1];
     x[0] = xl;
+}
+
+// f(k) for slots k = 0 .. NS - 1: with STOP until f returns false, else all of them
+template <int NS, bool STOP, typename F>
+__device__ __forceinline__ void each_slot(F &&f)
+{
+    if constexpr (STOP) {
+        static_while<0, NS>(f);
+    } else {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) (void)f(k);
+    }
 }
 
 // the value of lane `l` (the same in every lane)
@@ -853,6 +880,7 @@ __global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int 
             x[c][s] = (c < nc && r < n) ? x0[(long)c * n + r] : 0.0;
         }
     constexpr int D = NS == 1 ? 2 : 1;  // steps whose factor columns are loaded together
+    constexpr bool kStop = NS >= 4;     // leave a pass over the slots where the band ends
     // L solve with the interchanges, segment by segment (row j in slot 0)
 #pragma unroll 1
     for (int S = 0; S < NS; ++S) {
@@ -864,12 +892,17 @@ __global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int 
             for (int d = 0; d < D; ++d) {
                 const int j = j0 + d, lm = min(kl, n - 1 - j);
                 const double *col = ab + (long)j * ldab + kv - j;  // col[r] = factor entry (r, j)
-#pragma unroll
-                for (int k = 0; k < NS; ++k) {
+                auto load = [&](int k) {
                     const int r = (S + k) * 64 + lane;
-                    if (NS >= 8 && ((S + k) * 64 + 63 <= j || (S + k) * 64 > j + lm)) continue;
                     a[d][k] = j < jend && r > j && r <= j + lm ? col[r] : 0.0;
-                }
+                };
+                if constexpr (NS == 1) load(0);
+                else
+                    static_while<0, NS>([&](auto k) {
+                        if (kStop && (S + k) * 64 > j + lm) return false;
+                        load(k);
+                        return true;
+                    });
             }
         };
 #pragma unroll 1
@@ -886,9 +919,9 @@ __global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int 
 #pragma unroll
                 for (int c = 0; c < CPL; ++c) y[c] = lane_value(x[c][0], jj);
                 if (l != j)
-                    static_steps<0, NS>([&](auto slot) {
+                    static_while<0, NS>([&](auto slot) {
                         constexpr int k = decltype(slot)::value;
-                        if (k != lrel) return;
+                        if (k != lrel) return true;
                         asm volatile("" ::"n"(k));  // keeps the slots' branches apart: x[lrel] would put x into memory
 #pragma unroll
                         for (int c = 0; c < CPL; ++c) {
@@ -897,17 +930,21 @@ __global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int 
                             if (lane == (l & 63)) x[c][k] = y[c];
                             y[c] = xl;
                         }
+                        return false;
                     });
                 const int klo = ((j + 1) >> 6) - S, khi = ((j + lm) >> 6) - S;
+                each_slot<NS, kStop>([&](auto slot) {
+#pragma clang fp contract(off)
+                    const int k = slot, r = (S + k) * 64 + lane;
+                    if (kStop && k > khi) return false;
+                    if (!kStop && (k < klo || k > khi)) return true;
+                    if (r > j && r <= j + lm) {
 #pragma unroll
-                for (int k = 0; k < NS; ++k) {
-                    if (k < klo || k > khi) continue;
-                    const int r = (S + k) * 64 + lane;
-                    if (r <= j || r > j + lm) continue;
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c)
-                        if (y[c] != 0.0) x[c][k] = x[c][k] + a[d][k] * (-y[c]);
-                }
+                        for (int c = 0; c < CPL; ++c)
+                            if (y[c] != 0.0) x[c][k] = x[c][k] + a[d][k] * (-y[c]);
+                    }
+                    return true;
+                });
             });
         }
 #pragma unroll
@@ -926,13 +963,12 @@ __global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int 
                 const bool on = j >= 64 * S;
                 const double *col = ab + (long)j * ldab + kv - j;
                 dg[d] = on ? col[j] : 1.0;
-#pragma unroll
-                for (int k = 0; k < NS; ++k) {
-                    const int sa = k == 0 ? S : S - (NS - k);  // absolute slot of relative slot k
-                    const int r = sa * 64 + lane;
-                    if (NS >= 8 && (sa * 64 + 63 < lo || sa * 64 >= j)) continue;
+                each_slot<NS, kStop>([&](auto slot) {  // upwards from row j's
+                    const int i = slot, k = i == 0 ? 0 : NS - i, sa = S - i, r = sa * 64 + lane;
+                    if (kStop && sa * 64 + 63 < lo) return false;
                     a[d][k] = on && r >= lo && r < j ? col[r] : 0.0;
-                }
+                    return true;
+                });
             }
         };
         const int jtop = min(64 * S + 63, n - 1);
@@ -963,16 +999,18 @@ __global__ __launch_bounds__(64, NS == 8 ? 4 : 1) void band_lu_solve_kernel(int 
                     }
                 if (j == 0) return;
                 const int lo = max(0, j - kv), slo = lo >> 6, shi = (j - 1) >> 6;
+                each_slot<NS, kStop>([&](auto slot) {
+#pragma clang fp contract(off)
+                    const int i = slot, k = i == 0 ? 0 : NS - i, sa = S - i, r = sa * 64 + lane;
+                    if (kStop && sa < slo) return false;
+                    if (!kStop && (sa < slo || sa > shi)) return true;
+                    if (r >= lo && r < j) {
 #pragma unroll
-                for (int k = 0; k < NS; ++k) {
-                    const int sa = k == 0 ? S : S - (NS - k);
-                    if (sa < slo || sa > shi) continue;
-                    const int r = sa * 64 + lane;
-                    if (r < lo || r >= j) continue;
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c)
-                        if (nz[c]) x[c][k] = x[c][k] - t[c] * a[d][k];
-                }
+                        for (int c = 0; c < CPL; ++c)
+                            if (nz[c]) x[c][k] = x[c][k] - t[c] * a[d][k];
+                    }
+                    return true;
+                });
             });
         }
     }

@@ -46,3 +46,31 @@ def test_stp_of_unaligned_rows(ra, nt, near, lmax, nr, nf):
         s, p2 = zeros(plan.spectral_size), zeros(plan.hybrid_size)
         t.append(micros(lambda: plan.stp(s, p2)))
     assert t[0] <= 1.4 * t[1], t
+
+
+def band_problem(n, kl, nb, most):
+    """matrices of a diagonal that is mostly the pivot, most columns each"""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + kl)
+    ab = torch.zeros((nb, n, 3 * kl + 1), dtype=torch.float64, device="cuda")
+    ab[:, :, kl:] = torch.randn((nb, n, 2 * kl + 1), dtype=torch.float64, device="cuda", generator=g)
+    ab[:, :, 2 * kl] += 4.0 * (2 * kl) ** 0.5
+    i = torch.arange(n, device="cuda").view(n, 1) + torch.arange(3 * kl + 1, device="cuda").view(1, -1) - 2 * kl
+    ab[:, ~((i >= 0) & (i < n))] = 0.0
+    rhs = torch.randn(nb * most * n, dtype=torch.float64, device="cuda", generator=g)
+    off = torch.arange(nb, dtype=torch.int64, device="cuda") * (most * n)
+    return (ab.view(-1), torch.empty(nb * n, dtype=torch.int32, device="cuda"),
+            torch.empty(nb, dtype=torch.int32, device="cuda"), rhs, off,
+            torch.full((nb,), most, dtype=torch.int32, device="cuda"))
+
+
+@pytest.mark.parametrize("n,kl", [(1000, 4), (600, 40), (512, 2)])
+def test_band_solve_of_long_columns(ra, n, kl):
+    """A step's cost follows the band and not the column: a step of n = 1000, kl = 4 and of n = 600, kl
+    = 40 took twice as long as one of n = 250; 1.05 to 1.2 times now."""
+    t = []
+    for m in (n, 250):
+        a, piv, info, rhs, off, nc = band_problem(m, kl, 16, 8)
+        ra.lu_decompose_band(a, piv, info, m, kl)
+        t.append(micros(lambda: ra.lu_solve_band(a, piv, rhs, off, nc, m, kl, 8), reps=4) / m)
+    assert t[0] <= 1.6 * t[1], t
