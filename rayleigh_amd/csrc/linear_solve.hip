@@ -508,8 +508,25 @@ __global__ __launch_bounds__(kLuThreads) void lu_solve_lanes_kernel(int n, int n
         }
 }
 
-// Two right-hand sides per lane group: three waves per SIMD.  One costs 1.03 ms instead of 0.87 at
-// n = 256 (twice the LDS reads), three 1.07 and four 1.01 (fewer waves).
+// Two right-hand sides per lane group for n <= 512: three waves per SIMD.  One costs 1.03 ms instead
+// of 0.87 at n = 256 (twice the LDS reads), three 1.07 and four 1.01 (fewer waves).  For n > 512 the
+// staged columns (68 KB of LDS) leave a CU two workgroups whatever their registers are, and a
+// column's reads, which two lane groups of a wave shared below, serve one: every right-hand side
+// more costs a workgroup less than the last.  What counts is how many rounds of two workgroups on
+// 256 CUs a launch takes.  At n = 1000 (ms for 2 / 3 / 4 per group): one round with two, 64 matrices of 64
+// columns 1.40 / 1.69 / 1.55, 16 of 200 1.35 / 1.66 / 1.56; more, 64 of 2 (l + 1) (half of the groups
+// empty) 2.22 / 1.70 / 2.01, 64 of 200 4.60 / 4.16 / 3.89, 64 of 512 9.97 / 8.54 / 7.38; n = 513, 256 of 2 (l + 1)
+// 10.6 / 8.9 / 8.3.  So two as long as they fit one round, four from two rounds of fours on, three in between.
+constexpr long kSolveSlots = 512;
+
+// workgroups of a solve with cpl right-hand sides per group of G lanes
+template <int G>
+long lanes_workgroups(int cpl, int nbatch, int max_nrhs)
+{
+    const int cols = kLuThreads / G * cpl;
+    return (long)nbatch * ((max_nrhs + (long)cols - 1) / cols);
+}
+
 template <int G, int NT, int CPL>
 int launch_lanes(int n, int nbatch, const double *mats, const int *pivots, double *rhs, const long *rhs_off,
                  const int *nrhs, int max_nrhs, hipStream_t st)
@@ -1067,12 +1084,15 @@ int raysht_lu_solve_full(int n, int nbatch, const double *mats, const int *pivot
         rc = launch_lanes<16, 16, 2>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
     else if (n <= 512)
         rc = launch_lanes<32, 16, 2>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
-    else
+    else if (lanes_workgroups<64>(2, nbatch, max_nrhs) <= kSolveSlots)
         rc = launch_lanes<64, 16, 2>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
+    else if (lanes_workgroups<64>(4, nbatch, max_nrhs) < 2 * kSolveSlots)
+        rc = launch_lanes<64, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
+    else
+        rc = launch_lanes<64, 16, 4>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
     // a grid beyond the launch limit: fewer workgroups with three columns each
-    if (rc == RAYSHT_EUNSUPPORTED && n > 256)
-        rc = n <= 512 ? launch_lanes<32, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st)
-                      : launch_lanes<64, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
+    if (rc == RAYSHT_EUNSUPPORTED && n > 256 && n <= 512)
+        rc = launch_lanes<32, 16, 3>(n, nbatch, mats, pivots, rhs, rhs_off, nrhs, max_nrhs, st);
     if (rc != RAYSHT_OK) return rc;
     RAYSHT_HIP_TRY(hipGetLastError());
     return RAYSHT_OK;

@@ -74,3 +74,41 @@ def test_band_solve_of_long_columns(ra, n, kl):
         ra.lu_decompose_band(a, piv, info, m, kl)
         t.append(micros(lambda: ra.lu_solve_band(a, piv, rhs, off, nc, m, kl, 8), reps=4) / m)
     assert t[0] <= 1.6 * t[1], t
+
+
+def dense_columns(n, nb, cols):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + cols)
+    a = torch.randn((nb, n, n), dtype=torch.float64, device="cuda", generator=g)
+    a += 4.0 * n ** 0.5 * torch.eye(n, dtype=torch.float64, device="cuda")
+    rhs = torch.randn(nb * cols * n, dtype=torch.float64, device="cuda", generator=g)
+    off = torch.arange(nb, dtype=torch.int64, device="cuda") * (cols * n)
+    return (a.view(-1), torch.empty(nb * n, dtype=torch.int32, device="cuda"),
+            torch.empty(nb, dtype=torch.int32, device="cuda"), rhs, off,
+            torch.full((nb,), cols, dtype=torch.int32, device="cuda"))
+
+
+@pytest.mark.parametrize("n", [640, 1000])
+def test_dense_solve_of_many_columns(ra, n):
+    """512 columns of 64 matrices against 64: eight times the workgroups took 7.1 to 7.3 times as long;
+    fewer workgroups of more columns 5.3 to 5.6 times."""
+    t = []
+    for cols in (512, 64):
+        a, piv, info, rhs, off, nc = dense_columns(n, 64, cols)
+        ra.lu_decompose_full(a, piv, info, n)
+        t.append(micros(lambda: ra.lu_solve_full(a, piv, rhs, off, nc, n, cols), reps=3, tries=4))
+    assert t[0] <= 6.3 * t[1], t
+
+
+@pytest.mark.parametrize("n", [257, 300, 520])
+def test_dense_solve_of_a_huge_column_limit(ra, n):
+    """more workgroups than a launch may have with the fewest columns to each: nrhs is small, only the
+    limit that the caller gives is not; the solutions of an ordinary limit"""
+    import torch
+    a, piv, info, rhs, off, nc = dense_columns(n, 1, 5)
+    ra.lu_decompose_full(a, piv, info, n)
+    want = rhs.clone()
+    ra.lu_solve_full(a, piv, want, off, nc, n, 5)
+    most = 35_000_000 if n <= 512 else 24_000_000  # 2^24 workgroups are the most of 256 threads
+    ra.lu_solve_full(a, piv, rhs, off, nc, n, most)
+    assert torch.equal(rhs, want)
