@@ -589,13 +589,16 @@ __global__ __launch_bounds__(fft_geom<N>::THREADS, fft_geom<N>::WAVES) void fft_
 // share a line, each holds one butterfly of up to 16 points per stage in registers, and the
 // stages (two up to n2 = 240, three for most up to 2400) exchange through a padded LDS buffer of 8 bytes
 // per point, real parts and then imaginary parts.  The first stage reads the line from HBM,
-// the last stage of a c2r writes it there.  Lines of more than
-// 256 threads have an instance with radices up to 10 (MR), which fit the 128 VGPRs that workgroups of
-// up to 1024 threads leave.  (A Stockham in LDS with radices up to 8, two buffers of
-// 16 bytes per point and the first and last pass over LDS on their own ran at 0.8 - 1.7 TB/s;
-// this runs c2r at 1.9 - 4.0 and r2c at 2.2 - 4.9 where a line takes at most 256 threads, 1.2 - 2.2
-// above.  Only n2 = 1875 and 3675, odd and so no N_theta, got slower, by 11 and 27 % in c2r.)
-constexpr int kMaxRadix = 16, kMaxRadixSmall = 10, kMaxStages = 6;
+// the last stage of a c2r writes it there.  Lines of more than 256 threads take the instance (MR, threads)
+// whose registers let most waves share a CU: radices up to 10 fit the 128 VGPRs of four waves per
+// SIMD and so of workgroups up to 1024 threads; up to 6 (n2 = 1875, 3125, 3750) 72 VGPRs, and two or
+// three lines of 625 or 750 threads share a CU instead of one (1.6 GB of lines, c2r / r2c: n2 = 1875 2.60 /
+// 2.65 -> 1.58 / 1.54 ms, 3750 1.72 / 1.81 -> 1.06 / 1.08); n2 = 3675 alone needs a radix of 15 and 735 threads, and
+// gets 168 VGPRs and three waves per SIMD (at 128 its spills took 4.96 / 3.77 ms, now 1.92 / 2.09).
+// (A Stockham in LDS with radices up to 8, two buffers of 16 bytes per point and the first and
+// last pass over LDS on their own ran at 0.8 - 1.7 TB/s; this runs c2r at 1.9 - 4.0 and r2c at 2.2 - 4.9
+// where a line takes at most 256 threads, 1.2 - 3.0 above.)
+constexpr int kMaxRadix = 16, kMaxRadixLong = 10, kMaxRadixLow = 6, kMaxStages = 6;
 
 // Division of 0 <= x < 2^16 by a d that every thread shares, 1 <= d <= 2^13, as one high
 // multiplication by m = ceil(2^32 / d): exact, since m d - 2^32 < d and x d < 2^32.
@@ -707,7 +710,7 @@ __device__ __forceinline__ void any_stages(const any_sched &a, cplx (&v)[MR], an
 }
 
 template <bool C2R, int THREADS, int MR>
-__global__ __launch_bounds__(THREADS, (THREADS == 256 ? 3 : 4)) void fft_any_kernel(any_sched a, long howmany,
+__global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixLong ? 4 : 3)) void fft_any_kernel(any_sched a, long howmany,
                                                                                 double *__restrict__ x,
                                                                                 const double2 *__restrict__ tw,
                                                                                 int rescale)
@@ -1280,7 +1283,8 @@ int launch_hyb(const raysht_plan *p, const double *src, double *dst, const doubl
 // The schedule of fft_any_kernel for n2 = 2^a 3^b 5^c 7^d: the fewest stages of radix 2 .. 16, and
 // among those the one whose smallest radix is largest (fewest threads per line, all with a
 // full butterfly); where that takes more than 256 threads, the same with radices up to 10 if
-// 1024 threads suffice (they do for all but n2 = 3675).  False for other lengths.
+// 1024 threads suffice (they do for all but n2 = 3675, whose 735 threads have radices up to 15).
+// False for other lengths.
 bool any_schedule(int n2, bool c2r, any_sched *out)
 {
     static const int radices[] = {16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
@@ -1347,8 +1351,10 @@ int launch_any(int nphi, long howmany, double *x, const double2 *tw, int rescale
         hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), lds, st, a, howmany, x, tw, rescale);
     };
     if (threads <= 256) launch(fft_any_kernel<C2R, 256, kMaxRadix>);
-    else if (most <= kMaxRadixSmall) launch(fft_any_kernel<C2R, 1024, kMaxRadixSmall>);
-    else launch(fft_any_kernel<C2R, 1024, kMaxRadix>);
+    else if (most <= kMaxRadixLow && threads <= 768) launch(fft_any_kernel<C2R, 768, kMaxRadixLow>);
+    else if (most <= kMaxRadixLong && threads <= 1024) launch(fft_any_kernel<C2R, 1024, kMaxRadixLong>);
+    else if (threads <= 768) launch(fft_any_kernel<C2R, 768, kMaxRadix>);
+    else return RAYSHT_EUNSUPPORTED;  // no length's schedule
     RAYSHT_HIP_TRY(hipGetLastError());
     return RAYSHT_OK;
 }

@@ -112,3 +112,14 @@ def test_dense_solve_of_a_huge_column_limit(ra, n):
     most = 35_000_000 if n <= 512 else 24_000_000  # 2^24 workgroups are the most of 256 threads
     ra.lu_solve_full(a, piv, rhs, off, nc, n, most)
     assert torch.equal(rhs, want)
+
+
+@pytest.mark.parametrize("n2", [1875, 3675])
+def test_long_lines_of_odd_lengths(ra, n2):
+    """192 MB of lines of N_phi / 2 = 1875 (3 5^4) and 3675 (3 5^2 7^2) against 2401 (7^4): c2r 1.9 and 3.7
+    times as long, r2c 1.9 and 2.7; 1.1 and 1.55, 1.1 and 1.45 now."""
+    t = []
+    for n in (n2, 2401):
+        x = zeros(24_000_000 // (2 * n + 2) * (2 * n + 2))
+        t.append((micros(lambda: ra.fft_to_physical(x, 2 * n), reps=8), micros(lambda: ra.fft_to_spectral(x, 2 * n), reps=8)))
+    assert t[0][0] <= 1.72 * t[1][0] and t[0][1] <= 1.72 * t[1][1], t
