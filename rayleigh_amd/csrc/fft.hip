@@ -573,6 +573,26 @@ __global__ __launch_bounds__(fft_geom<N>::THREADS, fft_geom<N>::WAVES) void fft_
         }
         reinterpret_cast<double2 *>(xl)[k] = make_double2(re, im);
     };
+    if constexpr (G::P == 24 && T <= 4) {
+        // each lane has its line nearly to itself: from one end to the other its stores fill one
+        // cache line after the next, in pairs from both ends they come back to each later (192 MB
+        // of lines, N = 24, 48, 96: 78, 73, 68 us in pairs, 75, 67, 62 in order; for P = 16 pairs are as
+        // fast or faster)
+        cplx xk[G::P / 2 + 1], xn[G::P / 2 + 1];
+#pragma unroll
+        for (int u = 0; u <= G::P / 2; ++u) {
+            group_barrier<2>(u);
+            const int k = u < G::P / 2 ? t + T * u : N / 2;
+            xk[u] = r2c_unpack(zk[u], zn[u], tw[k]);
+            xn[u] = r2c_unpack(zn[u], zk[u], tw[N - k]);
+        }
+#pragma unroll
+        for (int u = 0; u < G::P / 2; ++u) put(t + T * u, xk[u]);
+        if (t == 0) put(N / 2, xk[G::P / 2]);
+#pragma unroll
+        for (int u = G::P / 2 - 1; u >= 0; --u) put(N - t - T * u, xn[u]);
+        return;
+    }
 #pragma unroll
     for (int u = 0; u <= G::P / 2; ++u) {
         group_barrier<2>(u);
@@ -1228,16 +1248,29 @@ bool with_reg_length(int n2, F &&f)
 #undef RAYSHT_LENGTH
 }
 
+// LDS asked for and not used: where one to four threads take a line, a lane walks its own cache
+// lines, and the 16 or more lines of a wave fill half of the 32 KB of a CU's vector cache.  Five
+// waves on a CU instead of nine or twelve keep what they walk in it.  192 MB of lines, c2r / r2c
+// without it -> with it, us: N = 16 82 / 80 -> 78 / 70, 24 102 / 82 -> 88 / 75, 32 89 / 65 -> 75 / 62, 48 131 / 68
+// -> 100 / 67, 64 90 / 63 -> 62 / 60, 96 106 / 66 -> 88 / 62; 6 KB are too few, 26 KB too many for some.
+template <int N>
+constexpr size_t reg_spare_lds()
+{
+    return fft_geom<N>::T <= 4 ? 14000 : 0;
+}
+
 template <int N>
 int launch_reg(bool c2r, long howmany, double *x, const double2 *tw, int rescale, hipStream_t st)
 {
+    constexpr size_t spare = reg_spare_lds<N>();
     constexpr int threads = fft_geom<N>::THREADS, lpb = threads / fft_geom<N>::T;
     const long blocks = (howmany + lpb - 1) / lpb;
     if (blocks > 0x7fffffffL) return RAYSHT_EUNSUPPORTED;
     if (c2r)
-        hipLaunchKernelGGL(fft_reg_c2r_kernel<N>, dim3((unsigned)blocks), dim3(threads), 0, st, howmany, x, tw);
+        hipLaunchKernelGGL(fft_reg_c2r_kernel<N>, dim3((unsigned)blocks), dim3(threads), spare, st, howmany, x,
+                           tw);
     else
-        hipLaunchKernelGGL(fft_reg_r2c_kernel<N>, dim3((unsigned)blocks), dim3(threads), 0, st, howmany, x, tw,
+        hipLaunchKernelGGL(fft_reg_r2c_kernel<N>, dim3((unsigned)blocks), dim3(threads), spare, st, howmany, x, tw,
                            rescale);
     RAYSHT_HIP_TRY(hipGetLastError());
     return RAYSHT_OK;
