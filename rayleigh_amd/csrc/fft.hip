@@ -821,15 +821,23 @@ __global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixL
 // Lines per workgroup, in waves of 64 threads (even, at most 32 lines).  Measured over 1, 2, 4 and
 // 8 waves on 1.6 GB grids (GB/s of rows plus grid, c2r / r2c): T = 4: 1 (4376 / 4874; two 4240 /
 // 4588); T = 8: 2 (4316 / 4513; four 3672 / 3697); T = 16: c2r 2, r2c 4 (3487 / 3998; the other
-// way 3420 / 3759); T = 32: 4 (3706 / 4306; two 3386 / 2877); T >= 64: 8 (3065 / 3663 at N = 1536;
-// four 3007 / 2637), c2r of T >= 128: 4 (2722; eight 2415).  More lines make longer pieces of the
+// way 3420 / 3759); T = 32: 4 (3706 / 4306; two 3386 / 2877); T = 64: 8 (3065 / 3663;
+// four 3007 / 2637); T >= 128: 4 (c2r 2722; eight 2415).  More lines make longer pieces of the
 // hybrid rows (8 bytes a line), fewer leave more workgroups to overlap their phases.
+// Where rows and grid stay in the last-level cache the r2c of T = 16 and 64 is faster with half the
+// lines: the pieces merge there, and a small grid has workgroups for more CUs.  N = 384, us with 4 / 2
+// waves by MB of grid: 2.4 10.8 / 9.0, 38 21.0 / 18.9, 151 61 / 57, 302 133 / 143, 605 252 / 273; N = 1536 with
+// 8 / 4: 9.4 18.1 / 13.0, 38 23.4 / 22.5, 75 46 / 33, 151 76 / 63, 302 175 / 236, 604 310 / 470.  T = 32 is not (9.4
+// 11.4 / 9.7, 38 20.6 / 20.2, 151 61 / 63, 302 147 / 207), and T = 128 is as fast or faster with 4 waves
+// at any size (19 22 / 16, 75 53 / 36, 302 185 / 162, 1208 743 / 743).
+constexpr double kCachedGridBytes = 200e6;
 template <int N, bool C2R>
-__host__ __device__ constexpr int hyb_lines()
+__host__ __device__ constexpr int hyb_lines(bool cached = false)
 {
     constexpr int T = fft_geom<N>::T;
-    constexpr int W = T <= 4 ? 1 : T == 8 ? 2 : T == 16 ? (C2R ? 2 : 4) : T == 32 ? 4 : T >= 128 && C2R ? 4 : 8;
-    return W * 64 / T > 32 ? 32 : W * 64 / T < 2 ? 2 : W * 64 / T;
+    constexpr int W = T <= 4 ? 1 : T == 8 ? 2 : T == 16 ? (C2R ? 2 : 4) : T == 32 || T >= 128 ? 4 : 8;
+    const int w = cached && !C2R && (T == 16 || T == 64) ? W / 2 : W;
+    return w * 64 / T > 32 ? 32 : w * 64 / T < 2 ? 2 : w * 64 / T;
 }
 
 struct hyb_args {
@@ -945,15 +953,15 @@ __global__ __launch_bounds__((hyb_lines<N, true>() * fft_geom<N>::T),
     if (t == 0) reinterpret_cast<double2 *>(xl)[N] = make_double2(0.0, 0.0);
 }
 
-// r2c and 3b -> 2b; the grid is left unchanged
-template <int N>
-__global__ __launch_bounds__((hyb_lines<N, false>() * fft_geom<N>::T),
+// r2c and 3b -> 2b; the grid is left unchanged.  TB lines to a workgroup.
+template <int N, int TB>
+__global__ __launch_bounds__((TB * fft_geom<N>::T),
                                   fft_geom<N>::WAVES) void fft_reg_r2c_hyb_kernel(hyb_args a,
                                     const double *__restrict__ p3, double *__restrict__ p2,
                                     const double2 *__restrict__ tw)
 {
     using G = fft_geom<N>;
-    constexpr int T = G::T, TB = hyb_lines<N, false>(), NTH = TB * T, PPR = TB / 2;
+    constexpr int T = G::T, NTH = TB * T, PPR = TB / 2;
     extern __shared__ double hyb_lds[];
     int r, f, t0;
     if (!hyb_unit(a, r, f, t0, TB)) return;
@@ -1284,10 +1292,10 @@ bool reg_dispatch(int n2, bool c2r, long howmany, double *x, const double2 *tw, 
 
 // the fused kernels of one register-resident length (arguments checked): c2r from the hybrid
 // rows in `src` to the grid, or r2c from the grid to the hybrid rows
-template <int N, bool C2R>
-int launch_hyb(const raysht_plan *p, const double *src, double *dst, const double2 *tw, hipStream_t st)
+template <int N, bool C2R, int TB>
+int launch_hyb_lines(const raysht_plan *p, const double *src, double *dst, const double2 *tw, hipStream_t st)
 {
-    constexpr int TB = hyb_lines<N, C2R>(), NTH = TB * fft_geom<N>::T, P = fft_geom<N>::P;
+    constexpr int NTH = TB * fft_geom<N>::T, P = fft_geom<N>::P;
     constexpr int US = (P + 2) / 3, UL = P / 2;
     static_assert(TB % 2 == 0 && 2 * US * fft_geom<N>::T <= N && 2 * UL * fft_geom<N>::T <= N,
                   "a thread moves two theta of a row, pieces stay within a line's modes");
@@ -1304,13 +1312,22 @@ int launch_hyb(const raysht_plan *p, const double *src, double *dst, const doubl
     const size_t lds = (size_t)TB * fft_geom<N>::STRIDE * sizeof(double);
     const dim3 grid((unsigned)(8 * ((units + 7) / 8))), block(NTH);
     if constexpr (!C2R)
-        hipLaunchKernelGGL(fft_reg_r2c_hyb_kernel<N>, grid, block, lds, st, a, src, dst, tw);
+        hipLaunchKernelGGL((fft_reg_r2c_hyb_kernel<N, TB>), grid, block, lds, st, a, src, dst, tw);
     else if ((p->lmax + 1) * (TB / 2) <= US * NTH)
         hipLaunchKernelGGL((fft_reg_c2r_hyb_kernel<N, US>), grid, block, lds, st, a, src, dst, tw);
     else
         hipLaunchKernelGGL((fft_reg_c2r_hyb_kernel<N, UL>), grid, block, lds, st, a, src, dst, tw);
     RAYSHT_HIP_TRY(hipGetLastError());
     return RAYSHT_OK;
+}
+
+template <int N, bool C2R>
+int launch_hyb(const raysht_plan *p, const double *src, double *dst, const double2 *tw, hipStream_t st)
+{
+    constexpr int TB = hyb_lines<N, C2R>(), TBC = hyb_lines<N, C2R>(true);
+    if (TBC != TB && 8.0 * (2 * N + 2) * p->nt * p->nr * p->nf <= kCachedGridBytes)
+        return launch_hyb_lines<N, C2R, TBC>(p, src, dst, tw, st);
+    return launch_hyb_lines<N, C2R, TB>(p, src, dst, tw, st);
 }
 
 // The schedule of fft_any_kernel for n2 = 2^a 3^b 5^c 7^d: the fewest stages of radix 2 .. 16, and

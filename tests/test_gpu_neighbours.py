@@ -135,3 +135,14 @@ def test_short_lines_in_place(ra, n2):
         t.append((micros(lambda: ra.fft_to_physical(x, 2 * n)), micros(lambda: ra.fft_to_spectral(x, 2 * n))))
     assert t[0][0] <= 1.25 * t[1][0] or n2 == 24, t
     assert t[0][1] <= 1.3 * t[1][1], t
+
+
+@pytest.mark.parametrize("n2,most", [(384, 1.0), (1536, 0.9), (3072, 1.1)])
+def test_reform_of_one_radius(ra, n2, most):
+    """reform_to_spectral of a grid with one radius against reform_to_physical of the same grid, which is
+    launched by other rules: 1.08, 1.01 and 1.25 times as long; .9, .73 and .92 now."""
+    nt, lmax = 384, min(1023, 2 * n2 // 3 - 1)
+    plan = ra.LegendrePlan(nt, lmax, ra.m_values_balanced(lmax), 1, 1)
+    p2, p3 = zeros(plan.hybrid_size), zeros((2 * n2 + 2) * nt)
+    t = (micros(lambda: plan.reform_to_spectral(p3, p2, 2 * n2)), micros(lambda: plan.reform_to_physical(p2, p3, 2 * n2)))
+    assert t[0] <= most * t[1], t
