@@ -1256,6 +1256,19 @@ bool with_reg_length(int n2, F &&f)
 #undef RAYSHT_LENGTH
 }
 
+// f(first line, lines) for pieces of `howmany` lines whose launches stay below 2^32 threads in
+// all (`block` threads take `per_block` lines); the pieces start at a workgroup's first line
+template <typename F>
+int in_pieces(long howmany, int per_block, int block, F &&f)
+{
+    const long most = ((1L << 32) - 1) / block * per_block;
+    for (long at = 0; at < howmany; at += most) {
+        f(at, std::min(most, howmany - at));
+        RAYSHT_HIP_TRY(hipGetLastError());
+    }
+    return RAYSHT_OK;
+}
+
 // LDS asked for and not used: where one to four threads take a line, a lane walks its own cache
 // lines, and the 16 or more lines of a wave fill half of the 32 KB of a CU's vector cache.  Five
 // waves on a CU instead of nine or twelve keep what they walk in it.  192 MB of lines, c2r / r2c
@@ -1272,16 +1285,12 @@ int launch_reg(bool c2r, long howmany, double *x, const double2 *tw, int rescale
 {
     constexpr size_t spare = reg_spare_lds<N>();
     constexpr int threads = fft_geom<N>::THREADS, lpb = threads / fft_geom<N>::T;
-    const long blocks = (howmany + lpb - 1) / lpb;
-    if (blocks > 0x7fffffffL) return RAYSHT_EUNSUPPORTED;
-    if (c2r)
-        hipLaunchKernelGGL(fft_reg_c2r_kernel<N>, dim3((unsigned)blocks), dim3(threads), spare, st, howmany, x,
-                           tw);
-    else
-        hipLaunchKernelGGL(fft_reg_r2c_kernel<N>, dim3((unsigned)blocks), dim3(threads), spare, st, howmany, x, tw,
-                           rescale);
-    RAYSHT_HIP_TRY(hipGetLastError());
-    return RAYSHT_OK;
+    return in_pieces(howmany, lpb, threads, [&](long at, long lines) {
+        const dim3 grid((unsigned)((lines + lpb - 1) / lpb));
+        double *xa = x + at * (2L * N + 2);
+        if (c2r) hipLaunchKernelGGL(fft_reg_c2r_kernel<N>, grid, dim3(threads), spare, st, lines, xa, tw);
+        else hipLaunchKernelGGL(fft_reg_r2c_kernel<N>, grid, dim3(threads), spare, st, lines, xa, tw, rescale);
+    });
 }
 
 bool reg_dispatch(int n2, bool c2r, long howmany, double *x, const double2 *tw, int rescale, hipStream_t st, int *rc)
@@ -1393,20 +1402,19 @@ int launch_any(int nphi, long howmany, double *x, const double2 *tw, int rescale
 {
     any_sched a;
     if (!any_schedule(nphi / 2, C2R, &a)) return RAYSHT_EUNSUPPORTED;
-    const long blocks = (howmany + a.lines - 1) / a.lines;
-    if (blocks > 0x7fffffffL) return RAYSHT_EUNSUPPORTED;
     const size_t lds = sizeof(double) * (size_t)a.lines * any_stride(a.n2);
     const int threads = a.lines * a.threads_line, most = *std::max_element(a.radix, a.radix + kMaxStages);
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), lds, st, a, howmany, x, tw, rescale);
+        return in_pieces(howmany, a.lines, threads, [&](long at, long lines) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)((lines + a.lines - 1) / a.lines)), dim3(threads), lds, st, a, lines,
+                               x + at * (nphi + 2L), tw, rescale);
+        });
     };
-    if (threads <= 256) launch(fft_any_kernel<C2R, 256, kMaxRadix>);
-    else if (most <= kMaxRadixLow && threads <= 768) launch(fft_any_kernel<C2R, 768, kMaxRadixLow>);
-    else if (most <= kMaxRadixLong && threads <= 1024) launch(fft_any_kernel<C2R, 1024, kMaxRadixLong>);
-    else if (threads <= 768) launch(fft_any_kernel<C2R, 768, kMaxRadix>);
-    else return RAYSHT_EUNSUPPORTED;  // no length's schedule
-    RAYSHT_HIP_TRY(hipGetLastError());
-    return RAYSHT_OK;
+    if (threads <= 256) return launch(fft_any_kernel<C2R, 256, kMaxRadix>);
+    if (most <= kMaxRadixLow && threads <= 768) return launch(fft_any_kernel<C2R, 768, kMaxRadixLow>);
+    if (most <= kMaxRadixLong && threads <= 1024) return launch(fft_any_kernel<C2R, 1024, kMaxRadixLong>);
+    if (threads <= 768) return launch(fft_any_kernel<C2R, 768, kMaxRadix>);
+    return RAYSHT_EUNSUPPORTED;  // no length's schedule
 }
 
 // the fused 2a -> 3a and c2r of any length; false where a line takes more than 128 threads
