@@ -1116,13 +1116,14 @@ int raysht_lu_decompose_band(int n, int kl, int ku, int nbatch, double *mats, in
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // threads by the size of the rank-1 update: 256 / 512 / 1024 take .080 / .089 / .100 ms at n = 64,
     // kl = 20 (170 matrices), .208 / .186 / .225 at 128, 40, .552 / .420 / .433 at 192, 72 and
-    // 1.196 / .726 / .704 at 256, 96 (256 matrices)
-    if (cols * ld <= most && kl <= 24)
-        launch_band_lds<256>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
-    else if (cols * ld <= most && kl <= 80)
+    // 1.196 / .726 / .704 at 256, 96 (256 matrices); a launch stays below 2^32 threads in all
+    auto fits = [&](int threads) { return (long)nbatch * threads < (1L << 32); };
+    if (cols * ld <= most && kl > 80 && fits(1024))
+        launch_band_lds<1024>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (cols * ld <= most && kl > 24 && fits(512))
         launch_band_lds<512>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
     else if (cols * ld <= most)
-        launch_band_lds<1024>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+        launch_band_lds<256>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
     else
         hipLaunchKernelGGL(band_lu_decompose_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), 0, st, n, kl,
                            ku, ldab, mats, pivots, info);

@@ -34,3 +34,21 @@ def test_more_lines_than_a_launch_holds(ra):
     expect([2.0, 0.0, 2.0, 0.0])
     del x
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("nb,kl", [(2 ** 22 + 3, 81), (2 ** 23 + 3, 25)])
+def test_band_matrices_by_the_million(ra, nb, kl):
+    """as many matrices of one row as 1024 (kl > 80) and 512 (kl > 24) threads each would pass the limit"""
+    import torch
+    ldab = 2 * kl + 1
+    if torch.cuda.mem_get_info()[0] < 8 * nb * ldab + 4e9:
+        pytest.skip("too little device memory")
+    ab = torch.full((nb, ldab), 7.0, dtype=torch.float64, device="cuda")
+    ab[::3, kl] = 0.0  # the diagonal
+    want = ab.clone()
+    piv = torch.full((nb,), -5, dtype=torch.int32, device="cuda")
+    info = torch.full((nb,), -5, dtype=torch.int32, device="cuda")
+    ra.lu_decompose_band(ab.view(-1), piv, info, 1, kl, 0)
+    assert torch.equal(ab, want)
+    assert bool((piv == 1).all())
+    assert int(info[::3].min()) == 1 and int(info.sum()) == (nb + 2) // 3
