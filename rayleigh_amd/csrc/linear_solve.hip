@@ -672,12 +672,16 @@ __global__ __launch_bounds__(kLuThreads) void band_lu_decompose_kernel(int n, in
 // column j (L, final) to LDS and the band storage in one pass; then the rank-1 update, in
 // which a thread stays on one ring row and keeps its multiplier in a register.  The arithmetic,
 // its order and the pivot choice are the global-memory kernel's, so the factors and pivots
-// are the same doubles.  Used where the window fits one workgroup's LDS.
+// are the same doubles.  Used where the window fits one workgroup's LDS.  Where only the step's own
+// rows and columns do (SPARE = false), the next ones come in after the update, into the slots
+// that the step has done with, at the price of a fourth barrier and a load that is waited for:
+// n = 640, kl = 30, ku = 612 (32 matrices) 1.99 ms instead of 5.22 in global memory, 400, 63, 255 1.31
+// instead of 3.97.
 // What bounds it is the chain of a column's phases (LDS latency, the barriers), then the LDS
 // rate of the update (three accesses per element).  With seven barriers a step, four LDS accesses per element
 // and 256 threads at every size it took, ms, against now: 170 matrices of n = 192, kl = 72 .813, .420;
 // 128, 40 .377, .186; 64, 20 .167, .080; 256 of n = 256, kl = 96 1.37, .704; n = 512, kl = 8 1.38, .637.
-template <int NT>
+template <int NT, bool SPARE>
 __global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl, int ku, int ldab, int ld,
                                                                    double *__restrict__ mats,
                                                                    int *__restrict__ pivots, int *__restrict__ infos)
@@ -687,7 +691,7 @@ __global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl
     const int tid = threadIdx.x, lane = tid & 63;
     double *ab = mats + (long)blockIdx.x * ldab * n;
     int *piv = pivots + (long)blockIdx.x * n;
-    const int kv = ku + kl, R = kl + 2, C = kv + 2;
+    const int kv = ku + kl, R = kl + (SPARE ? 2 : 1), C = kv + (SPARE ? 2 : 1);  // ring rows and columns
 #define AB(i, j) ab[(long)((j) - 1) * ldab + ((i) - 1)]
     // the first window, rows 1 .. min(kl + 1, n) x columns 1 .. min(kv + 1, n); entries more than
     // ku above the diagonal are fill-in, zero at the start
@@ -695,18 +699,18 @@ __global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl
         const int nrw = min(kl + 1, n), ncl = min(kv + 1, n);
         for (int e = tid; e < nrw * ncl; e += NT) {
             const int row = 1 + e % nrw, col = 1 + e / nrw;
-            win[col * ld + row] = col - row > ku ? 0.0 : AB(kv + 1 + row - col, col);
+            win[col % C * ld + row % R] = col - row > ku ? 0.0 : AB(kv + 1 + row - col, col);
         }
     }
     __syncthreads();
     const int rs = tid % ld, g = tid / ld, G = NT / ld;  // the update's ring row and its columns g, g + G, ...
-    int info = 0, ju = 1, jr = 1, jc = 1;                // jr, jc: the ring row and column of j
+    int info = 0, ju = 1, jr = 1 % R, jc = 1 % C;        // jr, jc: the ring row and column of j
     for (int j = 1; j <= n; ++j) {
         // ring rows / columns at an offset below R / C from j
         auto ring_row = [&](int i) { return jr + i >= R ? jr + i - R : jr + i; };
         auto ring_col = [&](int c) { return jc + c >= C ? jc + c - C : jc + c; };
         const int km = min(kl, n - j), rn = j + kl + 1, cn = j + kv + 1;
-        const double in = rn <= n && j + 1 + tid <= min(cn, n) ? AB(kv + rn - j - tid, j + 1 + tid) : 0.0;
+        const double in = SPARE && rn <= n && j + 1 + tid <= min(cn, n) ? AB(kv + rn - j - tid, j + 1 + tid) : 0.0;
         double *colj = win + jc * ld;
         // the largest |a| with the lowest index among equals; NaNs never enter
         double best = -1.0;
@@ -758,13 +762,15 @@ __global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl
                 AB(kv + 1 + i, j) = l;
             }
         }
-        // row and column of the next step into the ring slots of row and column j - 1
-        const int nr = jr > 0 ? jr - 1 : R - 1, ncol = jc > 0 ? jc - 1 : C - 1;
-        if (rn <= n)
-            for (int c = tid; c <= min(kv, n - j - 1); c += NT)
-                win[ring_col(c + 1) * ld + nr] = c == tid ? in : AB(kv + rn - j - c, j + 1 + c);
-        if (cn <= n)
-            for (int i = 1 + tid; i <= min(kl, n - j); i += NT) win[ncol * ld + ring_row(i)] = 0.0;
+        // row j + kl + 1 and column j + kv + 1 into the ring slots nr and ncol
+        auto bring_in = [&](int nr, int ncol) {
+            if (rn <= n)
+                for (int c = tid; c <= min(kv, n - j - 1); c += NT)
+                    win[ring_col(c + 1) * ld + nr] = SPARE && c == tid ? in : AB(kv + rn - j - c, j + 1 + c);
+            if (cn <= n)
+                for (int i = 1 + tid; i <= min(kl, n - j); i += NT) win[ncol * ld + ring_row(i)] = 0.0;
+        };
+        if (SPARE) bring_in(jr > 0 ? jr - 1 : R - 1, jc > 0 ? jc - 1 : C - 1);  // those of row and column j - 1
         __syncthreads();
         int i = rs - jr;
         if (i < 0) i += R;
@@ -791,6 +797,10 @@ __global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl
             }
         }
         __syncthreads();
+        if (!SPARE) {  // those of row and column j
+            bring_in(jr, jc);
+            __syncthreads();
+        }
         if (++jr == R) jr = 0;
         if (++jc == C) jc = 0;
     }
@@ -798,12 +808,13 @@ __global__ __launch_bounds__(NT) void band_lu_decompose_lds_kernel(int n, int kl
 #undef AB
 }
 
-template <int NT>
+template <int NT, bool SPARE>
 void launch_band_lds(int n, int kl, int ku, int nbatch, double *mats, int ldab, int ld, int *pivots, int *info,
                      hipStream_t st)
 {
-    hipLaunchKernelGGL((band_lu_decompose_lds_kernel<NT>), dim3((unsigned)nbatch), dim3(NT),
-                       sizeof(double) * (size_t)ld * (kl + ku + 2), st, n, kl, ku, ldab, ld, mats, pivots, info);
+    const size_t columns = kl + ku + (SPARE ? 2 : 1);
+    hipLaunchKernelGGL((band_lu_decompose_lds_kernel<NT, SPARE>), dim3((unsigned)nbatch), dim3(NT),
+                       sizeof(double) * columns * ld, st, n, kl, ku, ldab, ld, mats, pivots, info);
 }
 
 // Banded solve: LU_Solve_Band (Linear_Solve.F90:1056-1086, dgbtrs 'N').  One wave solves CPL
@@ -1106,24 +1117,35 @@ int raysht_lu_decompose_band(int n, int kl, int ku, int nbatch, double *mats, in
     if (nbatch > 0 && (!mats || !pivots || !info)) return RAYSHT_EINVAL;
     if (kl + ku > kBandMaxKv) return RAYSHT_EUNSUPPORTED;
     if (nbatch == 0) return RAYSHT_OK;
-    // the LDS-window kernel where its window fits one workgroup's LDS; an odd distance between columns
-    // keeps the interchange of a row off the same banks
+    // the LDS-window kernel where its window fits one workgroup's LDS, with a row and a column
+    // to spare if it can; an odd distance between columns keeps the interchange of a row off the
+    // same banks
     int dev = 0, lds_max = 0;
     RAYSHT_HIP_TRY(hipGetDevice(&dev));
     RAYSHT_HIP_TRY(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    const size_t cols = sizeof(double) * (size_t)(kl + ku + 2), most = (size_t)lds_max;
-    const int ld = cols * (size_t)((kl + 2) | 1) <= most ? (kl + 2) | 1 : kl + 2;
+    auto window = [&](int spare, int *ld) {
+        const long rows = kl + 1 + spare, room = lds_max / (8L * (kl + ku + 1 + spare));
+        *ld = (int)((rows | 1) <= room ? rows | 1 : rows);
+        return rows <= room;
+    };
+    int ld = 0;
+    const bool spare = window(1, &ld), tight = !spare && window(0, &ld);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // threads by the size of the rank-1 update: 256 / 512 / 1024 take .080 / .089 / .100 ms at n = 64,
     // kl = 20 (170 matrices), .208 / .186 / .225 at 128, 40, .552 / .420 / .433 at 192, 72 and
-    // 1.196 / .726 / .704 at 256, 96 (256 matrices); a launch stays below 2^32 threads in all
+    // 1.196 / .726 / .704 at 256, 96 (256 matrices), and without the spare row and column 3.09 / 2.18 /
+    // 1.99 at 640, 30, ku = 612 (32 matrices); a launch stays below 2^32 threads in all
     auto fits = [&](int threads) { return (long)nbatch * threads < (1L << 32); };
-    if (cols * ld <= most && kl > 80 && fits(1024))
-        launch_band_lds<1024>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
-    else if (cols * ld <= most && kl > 24 && fits(512))
-        launch_band_lds<512>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
-    else if (cols * ld <= most)
-        launch_band_lds<256>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    if (spare && kl > 80 && fits(1024))
+        launch_band_lds<1024, true>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (spare && kl > 24 && fits(512))
+        launch_band_lds<512, true>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (spare)
+        launch_band_lds<256, true>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (tight && fits(1024))
+        launch_band_lds<1024, false>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
+    else if (tight)
+        launch_band_lds<256, false>(n, kl, ku, nbatch, mats, ldab, ld, pivots, info, st);
     else
         hipLaunchKernelGGL(band_lu_decompose_kernel, dim3((unsigned)nbatch), dim3(kLuThreads), 0, st, n, kl,
                            ku, ldab, mats, pivots, info);
