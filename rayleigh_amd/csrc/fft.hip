@@ -1360,6 +1360,9 @@ bool any_schedule(int n2, bool c2r, any_sched *out)
             return;
         }
         if (depth >= kMaxStages || depth >= nbest) return;
+        int reach = 1;  // what the stages left can make of radices up to radices[from]
+        for (int d = depth; d < std::min(nbest, kMaxStages) && reach < n; ++d) reach *= radices[from];
+        if (reach < n) return;
         for (int i = from; i < 13; ++i)
             if (n % radices[i] == 0) {
                 cur[depth] = radices[i];
@@ -1374,7 +1377,6 @@ bool any_schedule(int n2, bool c2r, any_sched *out)
     };
     if (!schedule(0)) return false;
     if (n2 > 256 * std::max(smallest, 1) && (!schedule(4) || n2 > 1024 * smallest)) schedule(0);
-    if (!out) return true;
     // n2 / radix threads have a butterfly of a stage, so the stages that move the line to and from
     // HBM get the two smallest radices: a c2r, which reads two values per point, starts with the
     // smallest (4 to 14 % faster), an r2c with the second smallest (2 to 4 % faster).
@@ -1446,8 +1448,11 @@ bool launch_any_hyb(const raysht_plan *p, int nphi, const double *p2, double *p3
 int check_fft_args(int nphi, long howmany, const double *x)
 {
     if (nphi < 2 || (nphi & 1) || howmany < 0 || (!x && howmany > 0)) return RAYSHT_EINVAL;
-    if (nphi / 2 > kMaxHalf) return RAYSHT_EUNSUPPORTED;
-    return any_schedule(nphi / 2, true, nullptr) ? RAYSHT_OK : RAYSHT_EUNSUPPORTED;
+    int n2 = nphi / 2;
+    if (n2 > kMaxHalf) return RAYSHT_EUNSUPPORTED;
+    for (int p : {2, 3, 5, 7})  // every such length up to kMaxHalf has a schedule
+        while (n2 % p == 0) n2 /= p;
+    return n2 == 1 ? RAYSHT_OK : RAYSHT_EUNSUPPORTED;
 }
 
 // the c2r of `howmany` lines with the twiddle table tw of nphi (arguments checked)
