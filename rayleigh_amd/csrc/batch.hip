@@ -1,8 +1,9 @@
 // Many independent Legendre problems (plans of different l_max, N_theta and column
 // counts) in one grouped launch per direction: the m-blocks of every plan are dealt
 // to the XCDs together, longest contraction first, and each work item names its
-// problem; the kernels read that problem's tables and sizes from a descriptor array
-// in device memory and its input / output pointers from the launch arguments.
+// problem.  An FP64 item holds its table pointers and sizes; the split kernels read
+// their problem's from a descriptor array in device memory.  Input and output pointers
+// come with the launch arguments.
 #include <algorithm>
 #include <new>
 #include <vector>
@@ -107,10 +108,13 @@ int raysht_batch_create(raysht_batch **out, raysht_plan *const *plans, int n_pla
     b->precision = plans[0]->precision;
     b->plans.assign(plans, plans + n_plans);
     std::vector<const raysht_plan *> cp(plans, plans + n_plans);
-    std::vector<prob_desc> desc(n_plans);
-    for (int i = 0; i < n_plans; ++i) desc[i] = plans[i]->desc;
     const bool fp64 = b->precision == RAYSHT_FP64;
-    int rc = upload(&b->d_desc, desc);
+    int rc = RAYSHT_OK;
+    if (!fp64) {
+        std::vector<prob_desc> desc(n_plans);
+        for (int i = 0; i < n_plans; ++i) desc[i] = plans[i]->desc;
+        rc = upload(&b->d_desc, desc);
+    }
     for (int dir = 0; dir < 2 && rc == RAYSHT_OK; ++dir)
         for (int c = 0; c < kSchedules && rc == RAYSHT_OK; ++c) {
             if (fp64) {

@@ -621,7 +621,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void stp_split_kernel(
     __shared__ int cexp[kTileC];
     const int mp = uniform(work[blockIdx.x].mp);
     if (mp < 0) return;
-    const int pi = uniform(work[blockIdx.x].pad) & 0xffff, c0 = uniform(work[blockIdx.x].c0);
+    const int pi = uniform(work[blockIdx.x].prob), c0 = uniform(work[blockIdx.x].c0);
     const prob_desc &P = probs[pi];
     const int nt = uniform(P.nt), nt2 = uniform(P.nt2), nrhs = uniform(P.nrhs);
     const long *frag_off = uniform(P.frag_stp_off);
@@ -756,7 +756,7 @@ __global__ __launch_bounds__(kThreads, F::I8 && F::NA < 6 ? 3 : kMinWaves) void 
     __shared__ int cexp[2][kTileC];
     const int mp = uniform(work[blockIdx.x].mp);
     if (mp < 0) return;
-    const int pi = uniform(work[blockIdx.x].pad) & 0xffff, c0 = uniform(work[blockIdx.x].c0);
+    const int pi = uniform(work[blockIdx.x].prob), c0 = uniform(work[blockIdx.x].c0);
     const prob_desc &P = probs[pi];
     const int nt = uniform(P.nt), nt2 = uniform(P.nt2), nrhs = uniform(P.nrhs);
     const long *frag_off = uniform(P.frag_pts_off);
@@ -997,7 +997,7 @@ __global__ __launch_bounds__(kWsThreads, 1) void stp_split_ws_kernel(
     __shared__ int cexp[kTileC];
     const int mp = uniform(work[blockIdx.x].mp);
     if (mp < 0) return;
-    const int pi = uniform(work[blockIdx.x].pad) & 0xffff, c0 = uniform(work[blockIdx.x].c0);
+    const int pi = uniform(work[blockIdx.x].prob), c0 = uniform(work[blockIdx.x].c0);
     const prob_desc &P = probs[pi];
     const int nt = uniform(P.nt), nt2 = uniform(P.nt2), nrhs = uniform(P.nrhs);
     const int m = uniform(uniform(P.mvals)[mp]), nl = uniform(P.lmax) - m + 1, ne = (nl + 1) >> 1, no = nl >> 1;
@@ -1121,7 +1121,7 @@ __global__ __launch_bounds__(kWsThreads, 1) void pts_split_ws_kernel(
     __shared__ int cexp[2][kTileC];
     const int mp = uniform(work[blockIdx.x].mp);
     if (mp < 0) return;
-    const int pi = uniform(work[blockIdx.x].pad) & 0xffff, c0 = uniform(work[blockIdx.x].c0);
+    const int pi = uniform(work[blockIdx.x].prob), c0 = uniform(work[blockIdx.x].c0);
     const prob_desc &P = probs[pi];
     const int nt = uniform(P.nt), nt2 = uniform(P.nt2), nrhs = uniform(P.nrhs);
     const int m = uniform(uniform(P.mvals)[mp]), nl = uniform(P.lmax) - m + 1, ne = (nl + 1) >> 1, no = nl >> 1;
@@ -1265,11 +1265,11 @@ std::vector<work_item> split_work(const std::vector<const raysht_plan *> &plans,
         const raysht_plan *p = plans[b.prob];
         const int nct = cdiv(p->nrhs, kTileC);
         std::vector<work_item> items;
-        for (int c = 0; c < nct; ++c) items.push_back(work_item{b.mp, 0, c * kTileC, b.prob});
+        for (int c = 0; c < nct; ++c) items.push_back(work_item{b.mp, c * kTileC, b.prob});
         blocks.push_back(std::move(items));
         cost.push_back(b.item * nct);
     }
-    return deal_to_xcds(blocks, cost, o.xcd_groups, work_item{-1, 0, 0, 0});
+    return deal_to_xcds(blocks, cost, o.xcd_groups, work_item{-1, 0, 0});
 }
 
 namespace {

@@ -28,13 +28,12 @@ struct dd_pair {
     double hi, lo;
 };
 
-// One unit of grouped-GEMM work of the split kernels: m-block mp, column tile start, and in
-// `pad` the problem index.  An item runs every row tile of its column tile.
+// One unit of grouped-GEMM work of the split kernels: m-block mp (-1: padding), column tile start
+// and problem index.  An item runs every row tile of its column tile.
 struct work_item {
     int mp;
-    int r0;
     int c0;
-    int pad;
+    int prob;
 };
 
 // One tile of the FP64 kernels: row tile start r0 (nodes for StP, parity-l for PtS), column
@@ -68,14 +67,11 @@ struct raysht_split {
     int *d_texp_pts = nullptr;
 };
 
-// Everything a contraction kernel reads about one problem (one plan), in device
-// memory, so that one grouped launch can cover the m-blocks of several problems: the
-// `pad` field of a work item selects the problem.
+// Everything a split kernel reads about one problem (one plan), in device memory, so that
+// one grouped launch can cover the m-blocks of several problems; a work item names its problem.
 struct prob_desc {
-    const double *pt_even, *pt_odd, *ip_even, *ip_odd;  // FP64 tables
-    const long *s_off, *te_off, *to_off;
+    const long *s_off;
     const int *mvals;
-    // split forms (null for FP64 plans)
     const long *frag_stp_off, *frag_pts_off, *exp_pts_off;
     const uint4 *tdig_stp, *tdig_pts;
     const int *texp_stp, *texp_pts;
@@ -111,7 +107,7 @@ struct raysht_plan {
     // staging buffers of the host-array entry points, allocated on first use
     double *d_stage_s = nullptr, *d_stage_p = nullptr;
     raysht::raysht_split split;  // used by the BF16X3 / BF16X6 forms only
-    raysht::prob_desc desc{};           // this plan as one problem of a grouped launch
+    raysht::prob_desc desc{};  // this plan as one problem of a grouped launch (split forms)
     raysht::prob_desc *d_desc = nullptr;
     // radial transposes: LM_Load_Balance's (l, mp) pairs, the pair index of every
     // (m-block, l) at lm_base[mp] + l - m, and the (mp, first l - m) tiles
@@ -180,11 +176,11 @@ int launch_stp_split_batch(int precision, const prob_desc *d_desc, const batch_i
                            int n_work, hipStream_t st);
 int launch_pts_split_batch(int precision, const prob_desc *d_desc, const batch_io &io, const work_item *work,
                            int n_work, hipStream_t st);
-// XCD-balanced work lists over the m-blocks of several problems (work_item.pad = index
-// into `plans`), for the FP64 and the split kernels
-// Schedule options of a work list: PtS half-height last tiles (FP64 kernels), and
-// whether whole m-blocks are kept on one XCD (else the items go out in LPT order and
-// the dispatcher spreads consecutive items over the XCDs).
+// XCD-balanced work lists over the m-blocks of several problems (an item's `prob` = index into
+// `plans`), for the FP64 and the split kernels.
+// Schedule options of a work list: PtS row tiles that end with the m-block's rows (FP64 kernels;
+// off: full tiles), and whether whole m-blocks are kept on one XCD (else the items go out in LPT
+// order and the dispatcher spreads consecutive items over the XCDs).
 struct sched_opts {
     bool half_tiles = true;
     bool xcd_groups = true;

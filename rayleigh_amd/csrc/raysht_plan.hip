@@ -205,13 +205,7 @@ namespace {
 prob_desc describe(const raysht_plan *p)
 {
     prob_desc d{};
-    d.pt_even = p->d_pt_even;
-    d.pt_odd = p->d_pt_odd;
-    d.ip_even = p->d_ip_even;
-    d.ip_odd = p->d_ip_odd;
     d.s_off = p->d_s_off;
-    d.te_off = p->d_te_off;
-    d.to_off = p->d_to_off;
     d.mvals = p->d_mvals;
     d.frag_stp_off = p->split.d_frag_stp_off;
     d.frag_pts_off = p->split.d_frag_pts_off;
@@ -330,7 +324,7 @@ int plan_create(raysht_plan **out, int lmax, int ntheta, const int *m_values, in
     if (rc == RAYSHT_OK && precision != RAYSHT_FP64) rc = split_plan_init(p);
     if (rc == RAYSHT_OK) rc = radial_plan_init(p);
     if (rc == RAYSHT_OK) rc = angular_plan_init(p);
-    if (rc == RAYSHT_OK) {
+    if (rc == RAYSHT_OK && precision != RAYSHT_FP64) {
         p->desc = describe(p);
         rc = device_upload(&p->d_desc, &p->desc, 1);
     }
