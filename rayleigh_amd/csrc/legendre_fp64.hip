@@ -37,18 +37,19 @@ __device__ __forceinline__ double4_t mfma_f64(double a, double b, double4_t c)
 // twelve loads and LDS writes per wave and chunk before), 16-byte loads, and the loads of
 // the next chunk issued among this chunk's MFMAs.  On one long contraction (K = 512) StP
 // went from 58 to 71 TFLOP/s (a register-only MFMA loop reaches 74) and PtS from 58 to 66.
-// l_max = 511, N_theta = 768, N_r = 192, 8 fields: StP 6.60 -> 5.48 ms, PtS 6.60 -> 5.78 ms
-// (57 / 54 TFLOP/s); without their stores and data loads the same kernels take 4.4 / 4.8 ms,
-// so what is left above the matrix time is mostly the 13 GB each direction moves.
+// l_max = 511, N_theta = 768, N_r = 192, 8 fields: StP 6.60 -> 5.64 ms, PtS 6.60 -> 5.80 ms
+// (55 / 53 TFLOP/s; 5.5 - 5.9 and 5.6 - 6.1 over several machines); without their stores and data
+// loads the same kernels take 4.4 / 4.8 ms, so what is left above the matrix time is mostly the
+// 13.8 and 19.1 GB that they move (13.3 GB at least).
 // Measured and not kept: 4-wave workgroups with 32 columns per wave (half the LDS reads,
 // same rate at K = 512, 3-7 % slower on the whole path), wave priorities per workgroup,
 // scheduling barriers after every StP step.
 constexpr int kFp64MinWaves = 4;
 
 // Raw buffer access: each dword of a load whose byte offset falls outside [0, bytes) reads 0
-// without touching memory (a 16-byte load may straddle the end), so tile edges need no branches.  The whole offset goes in
-// the VGPR operand: the SGPR offset of a buffer load is not range-checked.  A negative
-// offset reads as a huge unsigned one, so it is out of range too.
+// without touching memory (a 16-byte load may straddle the end), so tile edges need no
+// branches.  The whole offset goes in the VGPR operand: the SGPR offset of a buffer load is not
+// range-checked.  A negative offset reads as a huge unsigned one, so it is out of range too.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const double *base, long bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(base), (short)0, (int)bytes, 0x00020000);

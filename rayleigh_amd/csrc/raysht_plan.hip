@@ -133,20 +133,13 @@ std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, 
         blocks.push_back(std::move(items));
         cost.push_back(b.item * (exact ? (double)nblk / full : nrt) * nct);
     }
-    // In a long launch heavy and light m-blocks alternate, so that tiles bound by the matrix
-    // cores (long contractions) share the CUs with tiles bound by memory (short ones, which
-    // otherwise all run together at the end).  In a short one the longest tiles go first:
-    // the tail they leave would cost more.  Measured (StP / PtS ms): l_max = 511, N_r = 192, 8
-    // fields, 72 / 51 rounds: 6.00 / 6.25 -> 5.91 / 6.15; l_max = 255, N_r = 128, 12 / 9 rounds:
-    // 0.648 / 0.646 -> 0.644 / 0.639; a batch of 12 problems, 7 / 5 rounds: 0.546 / 0.547 ->
-    // 0.552 / 0.564.
-    double total = 0.0, longest = 0.0;
-    for (size_t i = 0; i < order.size(); ++i) {
-        total += cost[i];
-        longest = std::max(longest, order[i].item);
-    }
-    constexpr double kSlots = 512.0, kMixRounds = 8.0;  // two workgroups on each of 256 CUs
-    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{}, total >= kMixRounds * kSlots * longest);
+    // Longest first within an XCD also in long launches: heavy and light m-blocks in turn, so that
+    // tiles bound by the matrix cores share the CUs with tiles bound by memory, measured the same
+    // within its noise of 1 % from 2 to 72 rounds of workgroups (StP / PtS us, longest first and in turn:
+    // l_max = 169, N_r = 96, 6 fields, 3 rounds 115 / 138 and 114 / 135; l_max = 255, 128 x 8, 12 rounds 596 /
+    // 610 and 594 / 598; l_max = 383, 128 x 5, 17 rounds 1106 / 1101 and 1121 / 1101; l_max = 511, 192 x 8, 72
+    // rounds 5650 / 5870 and 5625 / 5856; l_max = 1023, 32 x 5, 36 rounds 4280 / 4635 and 4309 / 4630).
+    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{});
 }
 
 void set_last_hip_error(hipError_t e, const char *what)
