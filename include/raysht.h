@@ -281,7 +281,9 @@ int raysht_reform_to_physical(raysht_plan *plan, int nphi, const double *p2, dou
 int raysht_reform_to_spectral(raysht_plan *plan, int nphi, double *p3, double *p2, void *stream);
 /* Fused forms of the same steps (results identical to the separate calls):
  * StP then 2a->3a then c2r, and r2c then 3b->2b then PtS.  `work` is a hybrid
- * buffer the call may overwrite.  For nphi / 2 = 3 * 2^k (24 .. 3072, Rayleigh's
+ * buffer the call may overwrite.  The 2a->3a transpose runs inside the c2r kernel for
+ * nphi / 2 = 3 * 2^k (24 .. 3072), 2^k (16 .. 4096) and the other lengths whose lines take
+ * at most 128 threads (all up to 672, few above 1500).  For nphi / 2 = 3 * 2^k (Rayleigh's
  * nphi = 3 (l_max + 1)) the 3b->2b transpose runs inside the r2c kernel (the padded grid
  * is read once); p3 is then left unchanged by raysht_reform_to_spectral /
  * raysht_physical_to_spectral, which otherwise transform it in place. */
@@ -307,7 +309,8 @@ int raysht_spectral_to_physical_scratch(raysht_plan *plan, int nphi, const doubl
 /* The spectral -> physical -> spectral round trip (StP, 2a->3a, c2r, r2c, 3b->2b,
  * PtS: Sphere_Hybrid_Space.F90:111,143 / Sphere_Physical_Space.F90:115,215 around an
  * identity physical step) recorded once into a hipGraph on the given device buffers;
- * each launch replays all six kernels with one call.  The plan and buffers must
+ * each launch replays all of them (four kernels, five or six where a transpose is one of
+ * its own) with one call.  The plan and buffers must
  * outlive the graph.  No reference counterpart: the reference launches each step
  * from the host every time step. */
 typedef struct raysht_graph raysht_graph;

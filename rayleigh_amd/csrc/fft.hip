@@ -607,7 +607,7 @@ __global__ __launch_bounds__(fft_geom<N>::THREADS, fft_geom<N>::WAVES) void fft_
 // Every other length, n2 = 2^a 3^b 5^c 7^d <= 4096 (N_theta = 240, 288, 360, ... and odd ones).  The
 // schedule is a run-time one, but the shape is the same: T = n2 / (smallest radix) threads
 // share a line, each holds one butterfly of up to 16 points per stage in registers, and the
-// stages (two up to n2 = 240, three for most up to 2400) exchange through a padded LDS buffer of 8 bytes
+// stages (two for most lengths up to 240, three up to 2400) exchange through a padded LDS buffer of 8 bytes
 // per point, real parts and then imaginary parts.  The first stage reads the line from HBM,
 // the last stage of a c2r writes it there.  Lines of more than 256 threads take the instance (MR, threads)
 // whose registers let most waves share a CU: radices up to 10 fit the 128 VGPRs of four waves per
@@ -1239,8 +1239,8 @@ int get_twiddles(int nphi, const double2 **out, bool create = true)
 }
 
 // calls f(std::integral_constant<int, N>) for a length n2 = N with register-resident kernels
-// (3 * 2^k, 24 .. 3072, and 2^k, 16 .. 4096); false for other lengths, which the LDS Stockham kernels
-// take
+// (3 * 2^k, 24 .. 3072, and 2^k, 16 .. 4096); false for other lengths, which fft_any_kernel and
+// fft_any_c2r_hyb_kernel take
 template <typename F>
 bool with_reg_length(int n2, F &&f)
 {

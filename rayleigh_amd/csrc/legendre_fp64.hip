@@ -40,7 +40,7 @@ __device__ __forceinline__ double4_t mfma_f64(double a, double b, double4_t c)
 // l_max = 511, N_theta = 768, N_r = 192, 8 fields: StP 6.60 -> 5.64 ms, PtS 6.60 -> 5.80 ms
 // (55 / 53 TFLOP/s; 5.5 - 5.9 and 5.6 - 6.1 over several machines); without their stores and data
 // loads the same kernels take 4.4 / 4.8 ms, so what is left above the matrix time is mostly the
-// 13.8 and 19.1 GB that they move (13.3 GB at least).
+// 14.0 and 18.3 GB that they move (13.3 GB at least).
 // Measured and not kept: 4-wave workgroups with 32 columns per wave (half the LDS reads,
 // same rate at K = 512, 3-7 % slower on the whole path), wave priorities per workgroup,
 // scheduling barriers after every StP step.
