@@ -830,6 +830,9 @@ __global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixL
 // 8 / 4: 9.4 18.1 / 13.0, 38 23.4 / 22.5, 75 46 / 33, 151 76 / 63, 302 175 / 236, 604 310 / 470.  T = 32 is not (9.4
 // 11.4 / 9.7, 38 20.6 / 20.2, 151 61 / 63, 302 147 / 207), and T = 128 is as fast or faster with 4 waves
 // at any size (19 22 / 16, 75 53 / 36, 302 185 / 162, 1208 743 / 743).
+// The c2r keeps its lines at every size: with half of them grids below 10 MB take less (N = 384, 2.4 MB
+// 10.0 / 8.9 us, N = 1536, 9.4 MB 17.9 / 13.8), from 40 MB on they are even or slower (384, 302 MB 154 / 162,
+// 1536, 1208 MB 677 / 692).
 constexpr double kCachedGridBytes = 200e6;
 template <int N, bool C2R>
 __host__ __device__ constexpr int hyb_lines(bool cached = false)
