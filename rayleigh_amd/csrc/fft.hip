@@ -687,7 +687,31 @@ __device__ __forceinline__ void any_first(const any_sched &a, any_state &q, int 
     q.busy = on && t < q.m;
 }
 
-template <int MR>
+// A thread's points in groups of GROUP: load(r, i) of each point r = g + i < R of a group, then
+// use(r, i).  A group's loads go out together; with its use behind each load a thread waits for
+// them one by one, which a launch of few lines has nothing to hide behind.  With CLAMP (c2r, three
+// loads a point) a group is loaded whole and without a branch, point 0 again for those at and above
+// R, whose results mean nothing.  Groups of four in the workgroups of 256 threads: c2r / r2c of one
+// line of N_phi = 480 8.8 / 10.6 -> 7.2 / 9.1 us (7.2 is what the host takes for a launch), 192 MB of
+// them 101 / 104 -> 76 / 102, N_phi = 30 248 / 161 -> 192 / 160 (369 with CLAMP off); of one, as it was,
+// where a line takes more threads (N_phi/2 = 2625, 192 MB, c2r 268 -> 290 with four).
+template <int MR, int GROUP, bool CLAMP, typename L, typename U>
+__device__ __forceinline__ void any_points(int R, L &&load, U &&use)
+{
+    constexpr bool whole = CLAMP && GROUP > 1;
+#pragma unroll
+    for (int g = 0; g < MR; g += GROUP)
+        if (g < R) {
+#pragma unroll
+            for (int i = 0; i < GROUP; ++i)
+                if (g + i < MR && (whole || g + i < R)) load(whole && g + i >= R ? 0 : g + i, i);
+#pragma unroll
+            for (int i = 0; i < GROUP; ++i)
+                if (g + i < MR && (whole || g + i < R)) use(g + i, i);
+        }
+}
+
+template <int MR, int GROUP, bool CLAMP>
 __device__ __forceinline__ void any_stages(const any_sched &a, cplx (&v)[MR], any_state &q, int t, bool on,
                                            double *__restrict__ buf, const double2 *__restrict__ tw, int sign)
 {
@@ -695,12 +719,12 @@ __device__ __forceinline__ void any_stages(const any_sched &a, cplx (&v)[MR], an
         const int jq = a.by_ns[s](t), jm = t - jq * q.ns;
         if (s > 0 && q.busy) {
             const int step = 2 * (q.m / q.ns) * jm;  // jm nphi / (ns R); times r below nphi
-#pragma unroll
-            for (int r = 1; r < MR; ++r)
-                if (r < q.R) {
-                    const double2 w = tw[step * r];
-                    v[r] = cmul(v[r], cplx{w.x, sign * w.y});
-                }
+            double2 w[GROUP];
+            any_points<MR, GROUP, CLAMP>(
+                q.R, [&](int r, int i) { w[i] = tw[step * r]; },
+                [&](int r, int i) {
+                    if (r > 0) v[r] = cmul(v[r], cplx{w[i].x, sign * w[i].y});
+                });
         }
         any_dft(v, q.R, sign);
         q.base = jq * q.ns * q.R + jm;
@@ -730,10 +754,8 @@ __device__ __forceinline__ void any_stages(const any_sched &a, cplx (&v)[MR], an
 }
 
 template <bool C2R, int THREADS, int MR>
-__global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixLong ? 4 : 3)) void fft_any_kernel(any_sched a, long howmany,
-                                                                                double *__restrict__ x,
-                                                                                const double2 *__restrict__ tw,
-                                                                                int rescale)
+__global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixLong ? 4 : 3)) void fft_any_kernel(
+    any_sched a, long howmany, double *__restrict__ x, const double2 *__restrict__ tw, int rescale)
 {
     extern __shared__ double any_lds[];
     const int n2 = a.n2, T = a.threads_line, tid = threadIdx.x;
@@ -745,22 +767,29 @@ __global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixL
     cplx v[MR];
     any_state q;
     any_first(a, q, t, on);
+    constexpr int GROUP = THREADS == 256 ? 4 : 1;
 #pragma unroll
-    for (int r = 0; r < MR; ++r) {
-        v[r] = {0.0, 0.0};
-        if (r < q.R && q.busy) {
-            const int k = t + r * q.m;
-            const double2 xa = xl[k];
-            if constexpr (C2R) {
-                const double2 xb = xl[n2 - k];
+    for (int r = 0; r < MR; ++r) v[r] = {0.0, 0.0};
+    if (q.busy) {
+        double2 xa[GROUP], xb[GROUP], w[GROUP];
+        any_points<MR, GROUP, C2R>(
+            q.R,
+            [&](int r, int i) {
+                const int k = t + r * q.m;
+                xa[i] = xl[k];
+                if constexpr (C2R) {
+                    xb[i] = xl[n2 - k];
+                    w[i] = tw[k];
+                }
+            },
+            [&](int r, int i) {
                 // Im X_0 and Im X_{n2} do not enter
-                v[r] = c2r_pack(cplx{xa.x, k == 0 ? 0.0 : xa.y}, cplx{xb.x, k == 0 ? 0.0 : -xb.y}, tw[k]);
-            } else {
-                v[r] = {xa.x, xa.y};
-            }
-        }
+                const bool k0 = t + r * q.m == 0;
+                if constexpr (C2R) v[r] = c2r_pack(cplx{xa[i].x, k0 ? 0.0 : xa[i].y}, cplx{xb[i].x, k0 ? 0.0 : -xb[i].y}, w[i]);
+                else v[r] = {xa[i].x, xa[i].y};
+            });
     }
-    any_stages(a, v, q, t, on, buf, tw, C2R ? +1 : -1);
+    any_stages<MR, GROUP, C2R>(a, v, q, t, on, buf, tw, C2R ? +1 : -1);
     if constexpr (C2R) {
 #pragma unroll
         for (int r = 0; r < MR; ++r)
@@ -769,7 +798,9 @@ __global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixL
     } else {
         // X_k and X_{n2-k} for k = t + i T <= n2 / 2; T >= n2 / MR
         constexpr int kPairs = MR / 2 + 1;
+        constexpr int kTogether = GROUP > 1 ? 3 : 1;  // pairs whose twiddles are loaded together, as in any_points
         double kr[kPairs], nr[kPairs];
+        double2 wk[kTogether], wn[kTogether];
 #pragma unroll
         for (int part = 0; part < 2; ++part) {
 #pragma unroll
@@ -778,6 +809,13 @@ __global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixL
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < kPairs; ++i) {
+                if (kTogether > 1 && part == 1 && i % kTogether == 0 && 2 * (t + i * T) <= n2)
+#pragma unroll
+                    for (int j = 0; j < kTogether; ++j) {
+                        const int k = min(t + (i + j) * T, n2);
+                        wk[j] = tw[k];
+                        wn[j] = tw[n2 - k];
+                    }
                 const int k = t + i * T;
                 if (2 * k <= n2 && on) {
                     const double zk = buf[any_pad(k)], zn = buf[any_pad(k == 0 ? 0 : n2 - k)];
@@ -795,8 +833,8 @@ __global__ __launch_bounds__(THREADS, (MR == kMaxRadixLow ? 7 : MR == kMaxRadixL
                             xl[i2] = make_double2(re, im);
                         };
                         const cplx a0 = {kr[i], zk}, a1 = {nr[i], zn};
-                        put(k, r2c_unpack(a0, a1, tw[k]));
-                        if (2 * k != n2) put(n2 - k, r2c_unpack(a1, a0, tw[n2 - k]));
+                        put(k, r2c_unpack(a0, a1, kTogether > 1 ? wk[i % kTogether] : tw[k]));
+                        if (2 * k != n2) put(n2 - k, r2c_unpack(a1, a0, kTogether > 1 ? wn[i % kTogether] : tw[n2 - k]));
                     }
                 }
             }
@@ -1113,7 +1151,7 @@ __global__ __launch_bounds__(256, 3) void fft_any_c2r_hyb_kernel(any_sched a, hy
             v[r] = c2r_pack(cplx{v[r].re, k == 0 ? 0.0 : ia}, cplx{nre[r], k == 0 ? 0.0 : -ib}, tw[k]);
         }
     __syncthreads();
-    any_stages(a, v, q, t, on, buf, tw, +1);
+    any_stages<kMaxRadix, 4, true>(a, v, q, t, on, buf, tw, +1);
     if (!on) return;
     double2 *xl = reinterpret_cast<double2 *>(p3 + (((long)f * h.nt + t0 + li) * h.nr + r0) * (2L * n2 + 2));
 #pragma unroll
