@@ -692,8 +692,8 @@ __device__ __forceinline__ void any_first(const any_sched &a, any_state &q, int 
 // them one by one, which a launch of few lines has nothing to hide behind.  With CLAMP (c2r, three
 // loads a point) a group is loaded whole and without a branch, point 0 again for those at and above
 // R, whose results mean nothing.  Groups of four in the workgroups of 256 threads: c2r / r2c of one
-// line of N_phi = 480 8.8 / 10.6 -> 7.2 / 9.1 us (7.2 is what the host takes for a launch), 192 MB of
-// them 101 / 104 -> 76 / 102, N_phi = 30 248 / 161 -> 192 / 160 (369 with CLAMP off); of one, as it was,
+// line of N_phi = 480 8.8 / 10.6 -> 7.3 / 9.2 us (7.2 is what the host takes for a launch), 192 MB of
+// them 100 / 84 -> 75 / 82, N_phi = 30 248 / 161 -> 191 / 156 (c2r 369 with CLAMP off); of one, as it was,
 // where a line takes more threads (N_phi/2 = 2625, 192 MB, c2r 268 -> 290 with four).
 template <int MR, int GROUP, bool CLAMP, typename L, typename U>
 __device__ __forceinline__ void any_points(int R, L &&load, U &&use)
