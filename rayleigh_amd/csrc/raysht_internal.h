@@ -193,11 +193,12 @@ std::vector<work_item> split_work(const std::vector<const raysht_plan *> &plans,
 // of one m-block, which share its P_lm table and its input columns, run on one XCD
 // and hit in its L2; within an XCD the largest contractions come first.  The list
 // is interleaved so that workgroup b runs item b/8 of XCD b%8, padded with `empty`
-// items where XCD queues differ in length.  Without XCD groups the blocks' items are
-// concatenated in the same longest-first order.
+// items where XCD queues differ in length.  With `in_turn` an XCD's blocks are the longest
+// and the shortest ones left in turn.  Without XCD groups the blocks' items are concatenated
+// in the same longest-first order.
 template <typename Item>
 std::vector<Item> deal_to_xcds(const std::vector<std::vector<Item>> &blocks, const std::vector<double> &cost,
-                               bool xcd_groups, const Item &empty)
+                               bool xcd_groups, const Item &empty, bool in_turn = false)
 {
     constexpr int kXcds = 8;
     if (!xcd_groups) {
@@ -206,11 +207,19 @@ std::vector<Item> deal_to_xcds(const std::vector<std::vector<Item>> &blocks, con
         return w;
     }
     std::vector<std::vector<Item>> q(kXcds);
+    std::vector<std::vector<size_t>> of(kXcds);  // the blocks of each XCD, longest first
     std::vector<double> load(kXcds, 0.0);
     for (size_t i = 0; i < blocks.size(); ++i) {
         const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        q[x].insert(q[x].end(), blocks[i].begin(), blocks[i].end());
+        of[x].push_back(i);
         load[x] += cost[i];
+    }
+    for (int x = 0; x < kXcds; ++x) {
+        const size_t n = of[x].size();
+        for (size_t i = 0; i < n; ++i) {
+            const auto &b = blocks[of[x][!in_turn ? i : i % 2 == 0 ? i / 2 : n - 1 - i / 2]];
+            q[x].insert(q[x].end(), b.begin(), b.end());
+        }
     }
     size_t len = 0;
     for (auto &v : q) len = std::max(len, v.size());

@@ -133,13 +133,25 @@ std::vector<fp64_item> fp64_work(const std::vector<const raysht_plan *> &plans, 
         blocks.push_back(std::move(items));
         cost.push_back(b.item * (exact ? (double)nblk / full : nrt) * nct);
     }
-    // Longest first within an XCD also in long launches: heavy and light m-blocks in turn, so that
-    // tiles bound by the matrix cores share the CUs with tiles bound by memory, measured the same
-    // within its noise of 1 % from 2 to 72 rounds of workgroups (StP / PtS us, longest first and in turn:
-    // l_max = 169, N_r = 96, 6 fields, 3 rounds 115 / 138 and 114 / 135; l_max = 255, 128 x 8, 12 rounds 596 /
-    // 610 and 594 / 598; l_max = 383, 128 x 5, 17 rounds 1106 / 1101 and 1121 / 1101; l_max = 511, 192 x 8, 72
-    // rounds 5650 / 5870 and 5625 / 5856; l_max = 1023, 32 x 5, 36 rounds 4280 / 4635 and 4309 / 4630).
-    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{});
+    // In a long launch an XCD's longest and shortest m-blocks run in turn, so that tiles bound by the
+    // matrix cores share the CUs with tiles bound by memory, which otherwise all run together at the
+    // end; in a short one the tail that this leaves costs more.  Longest first -> in turn, us:
+    //   PtS, l_max = 255, N_r = 128, 8 fields, 9 rounds of workgroups 594 -> 578; 200 x 8, 14 rounds 924 -> 892;
+    //   383, 128 x 8, 20 rounds 1683 -> 1671; 511, 96 x 6, 19 rounds 2125 -> 2080; 192 x 8, 51 rounds 5650 -> 5595;
+    //   1023, 32 x 5, 25 rounds 4450 -> 4450;
+    //   StP, 255, 128 x 8, 12 rounds 591 -> 585; 200 x 8, 19 rounds 906 -> 918; 319, 96 x 6, 11 rounds 600 -> 608; 383,
+    //   128 x 8, 27 rounds 1693 -> 1721; 511, 192 x 8, 72 rounds 5440 -> 5417; 1023, 64 x 5, 60 rounds 8008 -> 7953;
+    //   fewer rounds, PtS, 127, 64 x 4, 0.6 rounds 30 -> 34; 96 x 8, 1.9 rounds 95 -> 97; a batch of 12
+    //   problems, 5 rounds 547 -> 564 (but 255, 128 x 6, 7 rounds 449 -> 438); StP, 255, 64 x 4, 3 rounds 146 ->
+    //   155; 169, 128 x 8, 5 rounds 205 -> 209.
+    // Above the line both directions together gain up to 2 %, but lose 1 % at 383 and 0.3 % at 1023, 32 x 5.
+    double total = 0.0, longest = 0.0;
+    for (size_t i = 0; i < order.size(); ++i) {
+        total += cost[i];
+        longest = std::max(longest, order[i].item);
+    }
+    constexpr double kSlots = 512.0, kRounds = 8.0;  // two workgroups on each of 256 CUs
+    return deal_to_xcds(blocks, cost, o.xcd_groups, fp64_item{}, total >= kRounds * kSlots * longest);
 }
 
 void set_last_hip_error(hipError_t e, const char *what)
